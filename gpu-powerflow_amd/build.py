@@ -39,6 +39,8 @@ COMMON = [
 SOURCES = {
     "nr_kernels.hip": ["-ffp-contract=off"],
     "lu_kernels.hip": [],
+    "sys_kernels.hip": [],
+    "sys_plan.cpp": [],
     "newton_solver.cpp": [],
     "batched_lu.cpp": [],
     "analyze.cpp": [],

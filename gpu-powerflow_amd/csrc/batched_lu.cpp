@@ -151,33 +151,6 @@ void BatchedLU::analyze(int n, const int* rp, const int* ci, const std::vector<i
         }
         tile_ptr_[size_t(P.num_levels)] = int(tiles.size());
         d_tiles = upload_vector(tiles, s);
-        // single-system arena (fronts in plan order: children first)
-        std::vector<int> soff(size_t(P.num_fronts), 0);
-        long long tot = 0;
-        for (int p = 0; p < P.num_fronts; ++p) {
-            soff[size_t(p)] = int(std::min<long long>(tot, 1LL << 30));
-            tot += (long long)P.fsz[p] * P.fsz[p];
-        }
-        sdims_ = kern::SingleDims{};
-        sdims_.total = tot;
-        sdims_.P = P.num_fronts;
-        sdims_.nnz = P.ent_ptr[size_t(P.num_fronts)];
-        sdims_.nch = P.child_ptr[size_t(P.num_fronts)];
-        sdims_.nasm = P.asm_ptr[size_t(P.num_fronts)];
-        sdims_.nrows = P.front_ptr[size_t(P.num_fronts)];
-        sdims_.n = n;
-        const size_t need = std::max(kern::single_lds_bytes(sdims_, int(front_bytes()), false),
-                                     kern::single_lds_bytes(sdims_, int(front_bytes()), true));
-        single_fits_ = tot < (1LL << 30) && need <= kern::kSingleLdsMax;
-        single_ = false;
-        if (single_fits_) {
-            d_soff = upload_vector(soff, s);
-            sdims_.soff = d_soff.as<int>();
-            single_store_.allocate(size_t(tot) * front_bytes());
-        } else {
-            d_soff.release();
-            single_store_.release();
-        }
     }
     CUPF_HIP(hipStreamSynchronize(s));
 
@@ -198,6 +171,7 @@ void BatchedLU::analyze(int n, const int* rp, const int* ci, const std::vector<i
     lu.gat_ptr = d_gptr.as<int>(); lu.gat_src = d_gsrc.as<int>(); lu.rhs_idx = d_ridx.as<int>();
 
     find_chains(s);
+    find_sys(opt.n_bus, rp, ci, perm, s);
 
     // The timed dense stage is one kernel: the tile kernel when any level
     // takes it, else the row-block Schur kernel, else the tier-2 LU groups.
@@ -272,11 +246,58 @@ void BatchedLU::analyze(int n, const int* rp, const int* ci, const std::vector<i
 
     // batch buffers are sized lazily for the new structure
     capBp_ = 0;
-    for (DeviceBuffer* b : {&arena0_, &arena1_, &ywork_, &upd_, &res_, &sing_, &uinv_}) b->release();
+    for (DeviceBuffer* b : {&arena0_, &arena1_, &ywork_, &upd_, &res_, &sing_, &uinv_, &store_})
+        b->release();
     use_reserved();
     n_ = n;
     nnz_ = nnz;
 }
+
+// Panel cap of the one-workgroup plan: its fronts are blocked by 16 pivots
+// whatever their width, so wide panels only save levels.
+constexpr int kSysCap = 64;
+
+// Largest batch of the one-workgroup kernels.  They run a scenario per
+// workgroup, one to seven workgroups to a CU by their LDS, so their time grows
+// by the rounds of workgroups; the level sweeps cost some 0.5 ms a Newton step
+// however small the batch, and less per scenario once it is large.  Solves of
+// 250 buses mixed (one workgroup per CU): x1,024 2.05 against 3.12 ms, x1,536
+// 3.00 against 3.41, x2,048 4.6 against 3.9; 118 buses mixed (two): x2,048 1.60
+// against 2.38; 30 buses FP64 (seven): x2,048 0.71 against 1.05, x4,096 1.28
+// against 1.16.  The line lies where every measured shape gains.
+constexpr int kSysPerCu = 1024, kSysEver = 2048;
+
+void BatchedLU::find_sys(int n_bus, const int* rp, const int* ci, const std::vector<int>& perm,
+                         hipStream_t s) {
+    sys_ = SysPlan{};
+    sys_dev_ = kern::SysDevice{};
+    // fronts only grow with the cap, so a narrower plan's tell already
+    if (opt_.cap <= kSysCap && plan_.max_fsz > kSysMaxRows) return;
+    const LuPlan P = opt_.cap == kSysCap ? plan_ : lower_plan(analyze_symbolic(sym_.n, rp, ci, perm, kSysCap), sym_.n, rp, ci);
+    sys_ = make_sys_plan(P, kern::kSysLdsMax / front_bytes());
+    sys_lds_ = kern::sys_lds_bytes(sys_, int(front_bytes()), 0);
+    if (!sys_.ok || kern::sys_lds_bytes(sys_, int(front_bytes()), n_bus) > kern::kSysLdsMax) {
+        sys_.ok = false;
+        return;
+    }
+    const size_t lds = kern::sys_lds_bytes(sys_, int(front_bytes()), n_bus);
+    sys_most_ = int(std::min<size_t>(kSysEver, kSysPerCu * (kern::kSysLdsMax / lds)));
+    kern::sys_prepare();
+    d_sys_blob = upload_vector(sys_.blob, s);
+    d_sys_slot = upload_vector(sys_.slot_pos, s);
+    d_sys_adds = upload_vector(sys_.adds, s);
+    CUPF_HIP(hipStreamSynchronize(s));
+    kern::SysDevice& d = sys_dev_;
+    d.n = sys_.n; d.nnz = sys_.nnz; d.fac = sys_.fac; d.scratch = sys_.scratch;
+    d.blob_quads = int(sys_.blob.size() / 4);
+    d.num_levels = sys_.num_levels;
+    d.o_level = sys_.o_level; d.o_slice = sys_.o_slice; d.o_task = sys_.o_task;
+    d.o_rows = sys_.o_rows; d.o_gptr = sys_.o_gptr; d.o_gsrc = sys_.o_gsrc; d.o_perm = sys_.o_perm;
+    d.adds = d_sys_adds.as<unsigned short>();
+    d.blob = d_sys_blob.as<int4>();
+    d.slot_pos = d_sys_slot.as<int>();
+}
+
 
 // Chains of nested fronts (FP32 fronts; kern::chain_factor, nested_chains).
 // F0's own level is factored as usual, its pivot + Schur group writing the
@@ -419,16 +440,20 @@ size_t BatchedLU::uinv_elems(int Bp) const {
 
 namespace {
 // sizes of the batch buffers in LuBatchMem order
-void batch_parts(const LuPlan& P, int n, size_t ts, size_t uinv, int Bp, size_t out[7]) {
+constexpr int kParts = 8;
+// For Bp scenarios of the level sweeps, and sysBp of the one-workgroup kernels
+void batch_parts(const LuPlan& P, const SysPlan& sys, int n, size_t ts, size_t uinv, int Bp, int sysBp,
+                 size_t out[kParts]) {
     const size_t nb = size_t(Bp);
     out[0] = nb * std::max<size_t>(1, size_t(P.arena0)) * ts;
     out[1] = nb * std::max<size_t>(1, size_t(P.arena1)) * ts;
     out[2] = nb * size_t(n) * ts;
     // interleaved (tier-0 fronts) then scenario-major (tier-1/2 fronts)
     out[3] = 2 * nb * std::max<size_t>(1, size_t(P.upd_total)) * ts;
-    out[4] = nb * size_t(n) * sizeof(double);
-    out[5] = nb * sizeof(int);
-    out[6] = uinv * ts;
+    out[4] = std::max(nb, size_t(sysBp)) * size_t(n) * sizeof(double);
+    out[5] = std::max(nb, size_t(sysBp)) * sizeof(int);
+    out[6] = Bp > 0 ? uinv * ts : 0;
+    out[7] = sysBp > 0 ? size_t(sysBp) * kern::sys_store_elems(sys) * ts : 0;
 }
 constexpr size_t kPartAlign = 256;
 size_t align_up(size_t x) { return (x + kPartAlign - 1) / kPartAlign * kPartAlign; }
@@ -441,10 +466,12 @@ bool BatchedLU::reserve(int Bp) {
         use_reserved();
         return false;
     }
-    size_t sz[7];
-    batch_parts(plan_, n_, front_bytes(), uinv_elems(Bp), Bp, sz);
-    DeviceBuffer* own[7] = {&arena0_, &arena1_, &ywork_, &upd_, &res_, &sing_, &uinv_};
-    for (int i = 0; i < 7; ++i) {
+    // a batch that outgrows the one-workgroup kernels keeps room for smaller ones
+    size_t sz[kParts];
+    batch_parts(plan_, sys_, n_, front_bytes(), uinv_elems(Bp), sys_batch(Bp) ? 0 : Bp,
+                sys_.ok ? std::min(Bp, sys_most_) : 0, sz);
+    DeviceBuffer* own[kParts] = {&arena0_, &arena1_, &ywork_, &upd_, &res_, &sing_, &uinv_, &store_};
+    for (int i = 0; i < kParts; ++i) {
         if (sz[i]) own[i]->allocate(sz[i]);
         else own[i]->release();
     }
@@ -454,24 +481,27 @@ bool BatchedLU::reserve(int Bp) {
 }
 
 size_t BatchedLU::batch_bytes(int Bp) const {
-    size_t sz[7], total = 0;
-    batch_parts(plan_, n_, front_bytes(), uinv_elems(Bp), Bp, sz);
+    size_t sz[kParts], total = 0;
+    batch_parts(plan_, sys_, n_, front_bytes(), uinv_elems(Bp), sys_batch(Bp) ? 0 : Bp,
+                sys_batch(Bp) ? Bp : 0, sz);
     for (size_t v : sz) total += align_up(v);
     return total;
 }
 
 LuBatchMem BatchedLU::carve(void* base, int Bp) const {
-    size_t sz[7];
-    batch_parts(plan_, n_, front_bytes(), uinv_elems(Bp), Bp, sz);
+    size_t sz[kParts];
+    batch_parts(plan_, sys_, n_, front_bytes(), uinv_elems(Bp), sys_batch(Bp) ? 0 : Bp,
+                sys_batch(Bp) ? Bp : 0, sz);
     char* p = static_cast<char*>(base);
-    void* part[7];
-    for (int i = 0; i < 7; ++i) {
+    void* part[kParts];
+    for (int i = 0; i < kParts; ++i) {
         part[i] = sz[i] ? p : nullptr;
         p += align_up(sz[i]);
     }
     LuBatchMem m;
     m.arena0 = part[0]; m.arena1 = part[1]; m.ywork = part[2]; m.upd = part[3];
     m.res = static_cast<double*>(part[4]); m.sing = static_cast<int*>(part[5]); m.uinv = part[6];
+    m.store = part[7];
     return m;
 }
 
@@ -485,6 +515,7 @@ void BatchedLU::use_reserved() {
     mem_.arena0 = arena0_.get(); mem_.arena1 = arena1_.get(); mem_.ywork = ywork_.get();
     mem_.upd = upd_.get(); mem_.res = res_.as<double>(); mem_.sing = sing_.as<int>();
     mem_.uinv = uinv_.get();
+    mem_.store = store_.get();
     memBp_ = capBp_;
 }
 
@@ -628,14 +659,14 @@ void BatchedLU::factor_t(const double* A, int Bp, hipStream_t s, StageTimer* tim
 
 void BatchedLU::factor(const double* A, int Bp, hipStream_t s, StageTimer* timer, int stage) {
     if (Bp > memBp_) throw std::runtime_error("BatchedLU::factor(): batch exceeds the reserved size");
-    if (single_ && Bp == kern::kLanes) {
+    if (sys()) {
         const int sp = opt_.static_pivot ? 1 : 0;
         if (opt_.front64)
-            kern::single_factor<double>(lu_, sdims_, A, Bp, single_store_.as<double>(),
-                                        opt_.pivot_eps, sp, mem_.sing, s);
+            kern::sys_factor<double>(sys_dev_, A, B_, Bp, static_cast<double*>(mem_.store),
+                                     opt_.pivot_eps, sp, mem_.sing, sys_lds_, s);
         else
-            kern::single_factor<float>(lu_, sdims_, A, Bp, single_store_.as<float>(),
-                                       opt_.pivot_eps, sp, mem_.sing, s);
+            kern::sys_factor<float>(sys_dev_, A, B_, Bp, static_cast<float*>(mem_.store),
+                                    opt_.pivot_eps, sp, mem_.sing, sys_lds_, s);
         return;
     }
     if (opt_.front64) factor_t<double>(A, Bp, s, timer, stage);
@@ -676,13 +707,13 @@ void BatchedLU::solve_once(const double* rhs, TX* x, bool transpose, int Bp, hip
 
 template <typename TX>
 void BatchedLU::solve_dispatch(const double* rhs, TX* x, bool transpose, int Bp, hipStream_t s) {
-    if (single_ && Bp == kern::kLanes) {
+    if (sys()) {
         if (opt_.front64)
-            kern::single_solve<double, TX>(lu_, sdims_, single_store_.as<double>(), rhs, Bp, x,
-                                           transpose, s);
+            kern::sys_solve<double, TX>(sys_dev_, static_cast<const double*>(mem_.store), rhs,
+                                        B_, Bp, x, transpose, sys_lds_, s);
         else
-            kern::single_solve<float, TX>(lu_, sdims_, single_store_.as<float>(), rhs, Bp, x,
-                                          transpose, s);
+            kern::sys_solve<float, TX>(sys_dev_, static_cast<const float*>(mem_.store), rhs,
+                                       B_, Bp, x, transpose, sys_lds_, s);
         return;
     }
     if (opt_.front64) solve_once<double, TX>(rhs, x, transpose, Bp, s);

@@ -16,6 +16,7 @@
 #include "hip_common.hpp"
 #include "kernels.hpp"
 #include "stage_timer.hpp"
+#include "sys_kernels.hpp"
 
 #include <vector>
 
@@ -31,6 +32,7 @@ struct LuBatchMem {
     double* res = nullptr;
     int* sing = nullptr;
     void* uinv = nullptr;
+    void* store = nullptr;      // one-workgroup-per-system factors
 };
 
 struct LuOptions {
@@ -40,6 +42,8 @@ struct LuOptions {
     double pivot_eps = 1e-8;    // static pivot threshold and replacement magnitude
     bool static_pivot = true;   // replace small pivots (StaticDiagonalShift)
     bool chains = true;         // FP32 fronts: chains of nested fronts in one launch
+    int n_bus = 0;              // buses of the network whose Jacobian this is (0: none); the
+                                // one-workgroup kernels then keep its state in LDS too
 };
 
 class BatchedLU {
@@ -70,11 +74,14 @@ public:
     void use_memory(const LuBatchMem& mem, int Bp);
     void use_reserved();
 
-    // Batch-1 mode: with on and the whole factorisation fitting one wave's
-    // LDS, factor() and solve() at Bp == 64 run the single-system kernels on
-    // scenario 0 (solutions written to every lane).
-    void set_single(bool on) { single_ = on && single_fits_; }
-    bool single() const { return single_; }
+    // A pattern whose whole factorisation fits one workgroup's LDS runs the
+    // one-workgroup-per-system kernels while the batch is small enough
+    // (sys_most_).
+    bool sys() const { return sys_.ok && B_ > 0 && B_ <= sys_most_; }
+    const SysPlan& sys_plan() const { return sys_; }
+    const kern::SysDevice& sys_device() const { return sys_dev_; }
+    // Real scenarios of the following calls, which take Bp = B padded to 64.
+    void set_batch(int B) { B_ = B; }
 
     // Gates of the following launches (a captured Newton step run under a
     // device control word; null = open): the factor kernels set singular
@@ -84,11 +91,13 @@ public:
         gate_step_ = step;
         gate_refine_ = refine;
         lu_.gate = step;
+        sys_dev_.gate = step;
     }
 
     // Clear the per-scenario singular-pivot flags (a fill kernel).
     void clear_singular(int Bp, hipStream_t s);
     const int* singular() const { return mem_.sing; }
+    int* singular_flags() { return mem_.sing; }
 
     // Factor the values A [nnz][Bp] (interleaved FP64).  dense_timer, when
     // set, times the dense tier-2 launches under stage dense_stage.
@@ -134,6 +143,8 @@ private:
     bool tile_schur(int level) const;
     size_t uinv_elems(int Bp) const;
     void find_chains(hipStream_t s);
+    void find_sys(int n_bus, const int* rp, const int* ci, const std::vector<int>& perm, hipStream_t s);
+    bool sys_batch(int Bp) const { return sys_.ok && Bp <= sys_most_; }
     void split_tier1();
     template <typename T>
     void factor_t(const double* A, int Bp, hipStream_t s, StageTimer* timer, int stage);
@@ -179,17 +190,20 @@ private:
     std::vector<int> t2_max_uc_;
     std::vector<int> chain_at_;
     std::vector<char> chain_level_;
-    // single-system arena: front p at d_soff[p]
-    DeviceBuffer d_soff, single_store_;
-    kern::SingleDims sdims_;
-    bool single_fits_ = false, single_ = false;
+    // one-workgroup-per-system plan
+    SysPlan sys_;
+    DeviceBuffer d_sys_blob, d_sys_slot, d_sys_adds;
+    kern::SysDevice sys_dev_;
+    size_t sys_lds_ = 0;
+    int B_ = 0;
+    int sys_most_ = 0;            // largest batch that runs them, a multiple of 64
     // pattern and its transpose with value map (refinement residuals)
     DeviceBuffer d_rp, d_ci, d_trp, d_tci, d_tmap;
     kern::LuDevice lu_;
 
     // batch buffers: the reserved ones (capBp_) and the ones in use (memBp_)
     int capBp_ = 0;
-    DeviceBuffer arena0_, arena1_, ywork_, upd_, res_, sing_, uinv_;
+    DeviceBuffer arena0_, arena1_, ywork_, upd_, res_, sing_, uinv_, store_;
     LuBatchMem mem_;
     int memBp_ = 0;
 

@@ -947,6 +947,7 @@ int cupf_lu_factor(cupf_lu* h, const double* values, void* stream) {
         const hipStream_t s = stream ? static_cast<hipStream_t>(stream) : m.own;
         const int Bp = cupf::kern::pad_batch(m.B);
         cupf::kern::to_interleaved(values, m.nnz, m.nnz, m.B, Bp, m.A.as<double>(), s);
+        m.lu.set_batch(m.B);
         m.lu.clear_singular(Bp, s);
         m.lu.factor(m.A.as<double>(), Bp, s);
         m.factored = true;
@@ -962,6 +963,7 @@ static int lu_solve_common(cupf_lu* h, const double* rhs, double* x, void* strea
         const hipStream_t s = stream ? static_cast<hipStream_t>(stream) : m.own;
         const int Bp = cupf::kern::pad_batch(m.B);
         cupf::kern::to_interleaved(rhs, m.n, m.n, m.B, Bp, m.rhs.as<double>(), s);
+        m.lu.set_batch(m.B);
         m.lu.solve<double>(m.A.as<double>(), m.rhs.as<double>(), m.x.as<double>(),
                            m.xtmp.as<double>(), transpose, m.refine, Bp, s);
         cupf::kern::from_interleaved(m.x.as<double>(), m.n, m.B, Bp, x, m.n, s);
@@ -1010,6 +1012,7 @@ int cupf_lu_factor_solve_static(cupf_lu* h, int32_t batch, const double* values,
         m.lu.use_memory(m.lu.carve(base + vals + 3 * vec, Bp), Bp);
         cupf::kern::to_interleaved(values, m.nnz, m.nnz, batch, Bp, A, s);
         cupf::kern::to_interleaved(rhs, m.n, m.n, batch, Bp, b, s);
+        m.lu.set_batch(batch);
         m.lu.clear_singular(Bp, s);
         m.lu.factor(A, Bp, s);
         m.lu.solve<double>(A, b, xi, xt, transpose != 0, m.refine, Bp, s);

@@ -69,6 +69,15 @@ struct NewtonSolver::Impl {
         d_row_bus, d_row_isq;
     kern::NrDevice nr;
     BatchedLU lu;          // the Jacobian's batched multifrontal LU
+    // one-workgroup-per-system Newton steps (kern::sys_newton)
+    DeviceBuffer d_sys_ydst, d_sys_yrow, sys_sync;
+    kern::SysNet sys_net;
+    size_t sys_lds = 0;
+    // The loop runs on them when the system fits one workgroup; the FP32
+    // profile's state arithmetic and the stage timing have the separate
+    // kernels only.
+    bool sys_loop() const { return lu.sys() && !timer.on && nr.fp32_state == 0; }
+    bool seed_in_loop = false;        // the loop's first launch takes Va, Vm from V
 
     // batch buffers (scenario-interleaved, Bp = batch padded to 64)
     int capBp = 0, capB = 0;
@@ -124,8 +133,9 @@ struct NewtonSolver::Impl {
         const void* yb = nullptr;
         const void* head = nullptr;      // warm-start network of the head, if any
         unsigned long long gen = 0, head_gen = 0;
+        bool seed = false;               // the first launch takes Va, Vm from V
         bool operator==(const GraphKey& o) const {
-            return B == o.B && Bp == o.Bp && tolerant == o.tolerant && refine == o.refine &&
+            return seed == o.seed && B == o.B && Bp == o.Bp && tolerant == o.tolerant && refine == o.refine &&
                    limit == o.limit && steps == o.steps && pattern == o.pattern &&
                    tol == o.tol && yb == o.yb && head == o.head && gen == o.gen &&
                    head_gen == o.head_gen;
@@ -172,7 +182,7 @@ struct NewtonSolver::Impl {
         B = batch;
         Bp = kern::pad_batch(batch);
         if (lu.reserve(Bp)) ++buf_gen;
-        lu.set_single(batch == 1);
+        lu.set_batch(batch);
         if (Bp > capBp) {
             ++buf_gen;
             const size_t nb = size_t(Bp);
@@ -272,6 +282,7 @@ struct NewtonSolver::Impl {
         const int limit = budget >= 0 ? std::min(budget, cfg.max_iter) : cfg.max_iter;
         if (opt.use_cuda_graph && !timer.on && limit > 0)
             return run_nr_device(cfg, tolerant, limit, head, head_id, head_gen);
+        if (sys_loop() && limit > 0) return run_nr_sys(cfg, tolerant, limit, head);
         if (head) head();
         int completed = 0;
         for (int it = 0; it < limit; ++it) {
@@ -317,10 +328,68 @@ struct NewtonSolver::Impl {
         }
     };
 
+    // One launch of the one-workgroup Newton kernel.
+    void sys_launch(const NRConfig& cfg, bool tolerant, int limit, bool first, int steps,
+                    bool finish = false) {
+        kern::SysNewton o;
+        o.first = first;
+        o.seed = first && seed_in_loop;
+        o.finish = finish;
+        o.tolerant = tolerant;
+        o.steps = steps;
+        o.refine = refine;
+        o.limit = limit;
+        o.tol = cfg.tolerance;
+        o.refine_below = kRefineBelow;
+        auto go = [&](auto t) {
+            kern::sys_newton<decltype(t)>(lu.sys_device(), nr, sys_net, o, S.as<double2>(),
+                                          V.as<double2>(), Va.as<double>(), Vm.as<double>(),
+                                          normF.as<double>(), bmax.as<double>(), ctl.as<int>(),
+                                          sys_sync.as<unsigned long long>(), B, Bp, piv_eps,
+                                          static_piv ? 1 : 0, lu.singular_flags(), sys_lds, s);
+        };
+        if (front64) go(double());
+        else go(float());
+    }
+
+    // Steps enqueued before the first readback: a flat start takes 4 to 6, a
+    // launch on a stopped control word returns at once (2-3 us), a readback
+    // costs 15-20 us.
+    static constexpr int kSysAhead = 4;
+
+    // Eager loop on the one-workgroup kernel; the order and the outcome of
+    // the loop above, with one readback for several steps.
+    int run_nr_sys(const NRConfig& cfg, bool tolerant, int limit, const std::function<void()>& head) {
+        if (head) head();
+        int c[5] = {0, 0, 0, 0, 0};
+        double m = 0.0;
+        sys_launch(cfg, tolerant, limit, true, B == 1 ? limit - 1 : 0);
+        for (int k = 0; B > 1 && k < std::min(kSysAhead, limit - 1); ++k)
+            sys_launch(cfg, tolerant, limit, false, 1);
+        read_control(c, m);
+        while (!c[0]) {
+            sys_launch(cfg, tolerant, limit, false, 1);
+            read_control(c, m);
+        }
+        st.factorizations += c[2] - 1;
+        if (!tolerant && !std::isfinite(m))
+            throw std::runtime_error("NewtonSolver: mismatch norm is not finite");
+        if (!(m <= cfg.tolerance) && !(tolerant && m < 0.0)) {
+            // out of iterations: the loop ends with a step
+            sys_launch(cfg, tolerant, limit, false, 1, true);
+            ++st.factorizations;
+        }
+        return c[2];
+    }
+
     // Head of a device-run loop: initial V, residual, batch max, stop test.
     void loop_head(const std::function<void()>& head, const NRConfig& cfg, bool tolerant,
                    int limit) {
         if (head) head();
+        if (sys_loop()) {
+            sys_launch(cfg, tolerant, limit, true, B == 1 ? limit - 1 : 0);
+            return;
+        }
         eval_residual();
         enqueue_batch_max(tolerant);
         kern::nr_control(bmax.as<double>(), cfg.tolerance, kRefineBelow, refine, tolerant, limit,
@@ -333,6 +402,10 @@ struct NewtonSolver::Impl {
     // an unrefined step has none, and ctl[3] keeps its update, residual and
     // stop test from running when the device wants refinement.
     void loop_step(const NRConfig& cfg, bool tolerant, int limit, bool refined) {
+        if (sys_loop()) {                 // refined as the control word says
+            sys_launch(cfg, tolerant, limit, false, 1);
+            return;
+        }
         refined = refined && refine > 0;
         const int* step_gate = nullptr;
         {
@@ -415,13 +488,14 @@ struct NewtonSolver::Impl {
             const unsigned pattern =
                 refine > 0 ? pred_pattern[ti] & (steps >= 32 ? ~0u : (1u << steps) - 1u) : 0u;
             GraphKey key{B, Bp, ti, refine, limit, steps, pattern, cfg.tolerance, nr.yb, head_id,
-                         buf_gen, head_gen};
+                         buf_gen, head_gen, seed_in_loop};
             if (!solve_graphs[ti] || !(key == solve_keys[ti])) {
                 if (solve_graphs[ti]) (void)hipGraphExecDestroy(solve_graphs[ti]);
                 solve_graphs[ti] = nullptr;
                 solve_graphs[ti] = capture([&] {
                     loop_head(head, cfg, tolerant, limit);
-                    for (int k = 0; k < steps; ++k)
+                    // one scenario's first launch runs the whole loop
+                    for (int k = 0; k < (sys_loop() && B == 1 ? 0 : steps); ++k)
                         loop_step(cfg, tolerant, limit, k < 32 && ((pattern >> k) & 1u));
                 });
                 solve_keys[ti] = key;
@@ -488,6 +562,14 @@ struct NewtonSolver::Impl {
         nr.yb = Yb.as<double2>();
     }
 
+    // Va, Vm of the initial V
+    void seed(const NRConfig& cfg) {
+        seed_in_loop = sys_loop() && cfg.max_iter > 0;
+        if (!seed_in_loop)
+            kern::seed_polar(n, Bp, V.as<double2>(), Va.as<double>(), Vm.as<double>(), s,
+                             nr.fp32_state != 0);
+    }
+
     void solve_rows(const double2* Sr, int64_t ss, const double2* V0r, int64_t vs, int batch,
                     const NRConfig& cfg, bool cache_req, double2* Vo, std::vector<int>& iters,
                     std::vector<double>& nf, std::vector<int>& sg, const double2* Yr = nullptr,
@@ -498,8 +580,7 @@ struct NewtonSolver::Impl {
         load_ybus_rows(Yr, ys);
         if (!warm) {
             kern::to_interleaved(V0r, vs, n, B, Bp, V.as<double2>(), s);
-            kern::seed_polar(n, Bp, V.as<double2>(), Va.as<double>(), Vm.as<double>(), s,
-                             nr.fp32_state != 0);
+            seed(cfg);
             const int it = run_nr(cfg);
             if (cache_req) prepare_cache();
             kern::from_interleaved(V.as<double2>(), n, B, Bp, Vo, n, s);
@@ -531,8 +612,7 @@ struct NewtonSolver::Impl {
                 warm->predict_v0(Sh, sh, Rh, rh, B, warm_v0.as<double2>(), n, s);
             }
             kern::to_interleaved(warm_v0.as<double2>(), n, n, B, Bp, V.as<double2>(), s);
-            kern::seed_polar(n, Bp, V.as<double2>(), Va.as<double>(), Vm.as<double>(), s,
-                             nr.fp32_state != 0);
+            seed(cfg);
         };
         const int itw = run_nr(cfg, true, warm_budget, head, warm, warm->buffers_generation());
         kern::from_interleaved(V.as<double2>(), n, B, Bp, Vo, n, s);
@@ -563,8 +643,7 @@ struct NewtonSolver::Impl {
             if (Yr) load_ybus_rows(warm_y.as<double2>(), nnzY);
             kern::to_interleaved(warm_s.as<double2>(), n, n, B, Bp, S.as<double2>(), s);
             kern::to_interleaved(warm_r.as<double2>(), n, n, B, Bp, V.as<double2>(), s);
-            kern::seed_polar(n, Bp, V.as<double2>(), Va.as<double>(), Vm.as<double>(), s,
-                             nr.fp32_state != 0);
+            seed(cfg);
             const int itf = run_nr(cfg);
             kern::from_interleaved(V.as<double2>(), n, B, Bp, warm_o.as<double2>(), n, s);
             std::vector<double> nff;
@@ -770,6 +849,7 @@ void NewtonSolver::initialize(const YbusView& ybus, const int32_t* pv, int32_t n
     lo.cap = m.opt.custom.max_panel_width;
     lo.pivot_eps = m.piv_eps;
     lo.static_pivot = m.static_piv;
+    lo.n_bus = m.n;
     m.lu.analyze(m.js.dim, m.js.row_ptr.data(), m.js.col_idx.data(), perm, lo, m.own);
 
     hipStream_t s = m.own;
@@ -789,6 +869,26 @@ void NewtonSolver::initialize(const YbusView& ybus, const int32_t* pv, int32_t n
     m.d_zero = upload_vector(m.zero_slots, s);
     m.d_row_bus = upload_vector(m.js.row_bus, s);
     m.d_row_isq = upload_vector(m.js.row_is_q, s);
+    std::vector<int4> ydst;
+    std::vector<int> yrow;
+    m.sys_net = kern::SysNet{};
+    if (m.lu.sys_plan().ok) {
+        const std::vector<int>& pos = m.lu.sys_plan().slot_pos;
+        auto at = [&](int slot) { return slot >= 0 ? pos[size_t(slot)] : -1; };
+        for (int i = 0; i < m.n; ++i)
+            for (int k = m.yp[i]; k < m.yp[i + 1]; ++k) {
+                ydst.push_back(make_int4(at(m.js.map11[k]), at(m.js.map21[k]), at(m.js.map12[k]),
+                                         at(m.js.map22[k])));
+                yrow.push_back(i);
+            }
+        m.d_sys_ydst = upload_vector(ydst, s);
+        m.d_sys_yrow = upload_vector(yrow, s);
+        m.sys_sync.reserve(2 * sizeof(unsigned long long));
+        CUPF_HIP(hipMemsetAsync(m.sys_sync.get(), 0, 2 * sizeof(unsigned long long), s));
+        m.sys_net.ydst = m.d_sys_ydst.as<int4>();
+        m.sys_net.yrow = m.d_sys_yrow.as<int>();
+        m.sys_lds = kern::sys_lds_bytes(m.lu.sys_plan(), int(m.lu.front_bytes()), m.n);
+    }
     CUPF_HIP(hipStreamSynchronize(s));
 
     kern::NrDevice& nr = m.nr;
@@ -1093,6 +1193,7 @@ void NewtonSolver::solve_torch_forward(const void* sbus_base_re, const void* sbu
     m.bump();
     m.ensure_batch(batch_size);
     m.nr.yb = nullptr;   // Ybus values shared by the batch
+    m.seed_in_loop = false;
     const int B = m.B;
     if (want64)
         kern::torch_inputs<double>(m.n, B, m.Bp, (const double*)sbus_base_re,

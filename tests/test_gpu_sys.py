@@ -1,0 +1,112 @@
+"""One-workgroup-per-system kernels (sys_kernels.hip) against the oracle, at the
+sizes where their parts can go wrong: a grid of two buses, fronts at and
+around 16 and 32 rows (a quarter wave, a wave, the whole workgroup), the
+largest grids that fit one workgroup's LDS in FP64 and FP32 and the next ones
+that do not, and batches of one workgroup, one per CU and on either side of the
+hand-over to the level sweeps."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+import capi
+
+pytestmark = pytest.mark.gpu
+
+
+def _solver(cupf, g, compute, cap=64):
+    o = cupf.NewtonOptions()
+    o.compute = getattr(cupf.ComputePolicy, compute)
+    o.custom.precision = cupf.CustomPrecision.FP64 if compute == "FP64" else cupf.CustomPrecision.FP32
+    o.custom.max_panel_width = cap
+    s = cupf.NewtonSolver(o)
+    s.initialize(g.indptr, g.indices, g.data, g.n_bus, g.n_bus, g.pv, g.pq)
+    return s
+
+
+def _grid(syn, n, ratio=1.55):
+    return syn.make_grid(n, max(n - 1, int(n * ratio)) if n > 2 else 1, int(0.15 * n), seed=n,
+                         load_scale=min(0.25, 100.0 / n))
+
+
+# 2..40 buses: quarter-wave and wave fronts; 118: shared root; 150 / 175 FP64
+# and 250 / 320 mixed: either side of the LDS limit
+@pytest.mark.parametrize("compute,n,B", [
+    ("FP64", 2, 1), ("Mixed", 2, 3), ("FP64", 9, 65), ("FP64", 40, 257), ("Mixed", 40, 64),
+    ("FP64", 118, 1), ("FP64", 118, 300), ("Mixed", 118, 130), ("FP64", 150, 5), ("FP64", 175, 5),
+    ("Mixed", 250, 7), ("Mixed", 320, 7), ("FP64", 30, 2048), ("FP64", 30, 2049)])
+def test_solve_matches_oracle(gpu, cupf, syn, oracle, compute, n, B):
+    print(f"[sys] {compute} n={n} B={B}", flush=True)
+    g = _grid(syn, n)
+    S = g.sbus_scaled(syn.load_factors(B, n, 0.7, 1.3, 5))
+    V0 = g.flat_start(B)
+    r = _solver(cupf, g, compute).solve_batch(g.indptr, g.indices, g.data, n, n, S, V0, g.pv, g.pq)
+    k = min(B, 4)
+    pick = np.unique(np.r_[np.arange(k), B - 1])
+    Vo, io, _, _ = oracle.nr_solve_batch(n, g.indptr, g.indices, g.data, S[pick], V0[pick], g.pv, g.pq,
+                                         tol=1e-13)
+    assert r.converged_numpy.all()
+    # one further Newton step from ||F|| <= 1e-8 is quadratic; the state is
+    # within the tolerance times the inverse Jacobian's norm (below 10 here)
+    assert np.abs(r.V_numpy[pick] - Vo).max() <= 1e-7
+    assert (r.V_numpy[:, g.slack] == V0[:, g.slack]).all()
+
+
+@pytest.mark.parametrize("compute,tol", [("FP64", 1e-12), ("Mixed", 1e-9)])
+@pytest.mark.parametrize("n,B", [(2, 1), (30, 65), (118, 300), (150, 3)])
+@pytest.mark.parametrize("transpose", [False, True])
+def test_factor_solve(gpu, cupf, syn, oracle, compute, tol, n, B, transpose):
+    print(f"[sys] factor+solve {compute} n={n} B={B} transpose={transpose}", flush=True)
+    g = _grid(syn, n)
+    s = _solver(cupf, g, compute)
+    ja = oracle.jacobian_analysis(n, g.indptr, g.indices, g.pv, g.pq)
+    rng = np.random.default_rng(n)
+    V = rng.uniform(0.97, 1.03, (B, n)) * np.exp(1j * rng.uniform(-0.1, 0.1, (B, n)))
+    A = np.stack([oracle.jacobian_values(n, g.indptr, g.indices, g.data, v, g.pv, g.pq, ja["nnz"])
+                  for v in V[:5]])[np.arange(B) % 5]
+    rhs = rng.standard_normal((B, ja["dim"]))
+    x, sing = capi.debug_factor_solve(s.handle, A, rhs, transpose=transpose)
+    assert not sing.any()
+    for b in np.unique(np.r_[np.arange(min(B, 6)), B - 1]):
+        M = sp.csr_matrix((A[b], ja["col_idx"], ja["row_ptr"]), shape=(ja["dim"],) * 2)
+        M = M.T if transpose else M
+        assert np.linalg.norm(M @ x[b] - rhs[b]) <= tol * np.linalg.norm(rhs[b]), b
+
+
+def test_iteration_limits_match_the_level_sweeps(gpu, cupf, syn):
+    """Out of iterations the loop ends with a step, as the batched loop does
+    (2,049 scenarios run the level sweeps, 70 the one-workgroup kernels)."""
+    g = _grid(syn, 30)
+    S = g.sbus_scaled(syn.load_factors(2049, 30, 0.7, 1.3, 6))
+    V0 = g.flat_start(2049)
+    args = (g.indptr, g.indices, g.data, 30, 30)
+    s = _solver(cupf, g, "FP64")
+    for limit in (0, 1, 2, 3):
+        c = cupf.NRConfig()
+        c.max_iter = limit
+        for B in (1, 70):
+            a = s.solve_batch(*args, S[:B], V0[:B], g.pv, g.pq, c)
+            b = s.solve_batch(*args, S, V0, g.pv, g.pq, c)
+            assert (a.iterations_numpy == limit).all() and (b.iterations_numpy == limit).all()
+            np.testing.assert_allclose(a.V_numpy, b.V_numpy[:B], rtol=0, atol=1e-12)
+
+
+def test_small_pivots_are_replaced_and_flagged(gpu, cupf, syn, oracle):
+    """A zero diagonal entry of an isolated row: the static pivot rule, per
+    scenario."""
+    g = _grid(syn, 30)
+    s = _solver(cupf, g, "FP64")
+    ja = oracle.jacobian_analysis(30, g.indptr, g.indices, g.pv, g.pq)
+    A = np.zeros((70, ja["nnz"]))
+    rows = np.repeat(np.arange(ja["dim"]), np.diff(ja["row_ptr"]))
+    A[:, rows == ja["col_idx"]] = 2.0
+    d3 = np.flatnonzero((rows == 3) & (ja["col_idx"] == 3))[0]
+    A[7, d3] = 0.0
+    A[9, d3] = -1e-12
+    x, sing = capi.debug_factor_solve(s.handle, A, np.ones((70, ja["dim"])))
+    want = np.full((70, ja["dim"]), 0.5)
+    want[7, 3], want[9, 3] = 1e8, -1e8
+    np.testing.assert_allclose(x, want, rtol=1e-15)
+    assert sing[7] and sing[9] and sing.sum() == 2
