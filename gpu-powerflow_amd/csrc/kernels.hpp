@@ -78,6 +78,10 @@ void refine_residual(const int* rp, const int* ci, const int* vmap, const double
                      int Bp, const double* F, const TX* x, double* r, hipStream_t s);
 template <typename TX>
 void axpy_update(const TX* ddx, TX* dx, long long count, hipStream_t s, const int* gate = nullptr);
+// out[0 .. sum_squares_parts) = sums of v[i * Bp + b]^2 over blocks of rows and
+// scenarios b < B, in a fixed order; at most dim * Bp / 256 + 1 parts.
+int sum_squares_parts(int dim, int Bp);
+void sum_squares(const double* v, int dim, int B, int Bp, double* out, hipStream_t s);
 // max over scenarios b < B of normF[b] -> out[0]
 void batch_max(const double* normF, int B, double* out, hipStream_t s, const int* gate = nullptr);
 // the same over the finite entries only; -1 when none is finite

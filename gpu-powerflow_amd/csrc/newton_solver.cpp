@@ -689,6 +689,18 @@ struct NewtonSolver::Impl {
         CUPF_HIP(hipStreamSynchronize(s));
     }
 
+    // Host rows ([B][stride]) to packed device rows ([B][cols]).  Packed rows go
+    // in one copy: a 2D copy from pageable memory goes row by row, some 10 us
+    // each (a solve of 300 rows of 118 buses: 6.1 ms against 0.6).
+    void upload_rows(void* dst, const void* src, int64_t stride, int64_t cols, int rows, size_t elem) {
+        const size_t row = size_t(cols) * elem;
+        if (stride == cols || rows == 1)
+            CUPF_HIP(hipMemcpyAsync(dst, src, size_t(rows) * row, hipMemcpyHostToDevice, s));
+        else
+            CUPF_HIP(hipMemcpy2DAsync(dst, row, src, size_t(stride) * elem, row, rows,
+                                      hipMemcpyHostToDevice, s));
+    }
+
     void check_ybus(const YbusView& y) const {
         if (y.rows != n || y.cols != n || y.nnz != nnzY)
             throw std::runtime_error("NewtonSolver: Ybus dimensions do not match initialize()");
@@ -969,10 +981,8 @@ void NewtonSolver::solve_batch(const YbusView& ybus, const std::complex<double>*
     const int B = m.B;
     m.upload_ybus_values(ybus);
     const size_t row = size_t(m.n) * sizeof(double2);
-    CUPF_HIP(hipMemcpy2DAsync(m.stage_a.get(), row, sbus, size_t(sbus_stride) * sizeof(double2), row,
-                              B, hipMemcpyHostToDevice, m.s));
-    CUPF_HIP(hipMemcpy2DAsync(m.stage_b.get(), row, V0, size_t(V0_stride) * sizeof(double2), row, B,
-                              hipMemcpyHostToDevice, m.s));
+    m.upload_rows(m.stage_a.get(), sbus, sbus_stride, m.n, B, sizeof(double2));
+    m.upload_rows(m.stage_b.get(), V0, V0_stride, m.n, B, sizeof(double2));
     const bool cache_req = solve_options.prepare_adjoint_cache &&
                            solve_options.adjoint_cache_mode != AdjointCacheMode::None;
     std::vector<int> its, sing;
@@ -1103,10 +1113,8 @@ void NewtonSolver::solve_adjoint(const double* grad_va, int64_t grad_va_stride,
         result.jt_factorized_during_forward_cache = true;
     }
     const size_t row = size_t(m.n) * sizeof(double);
-    CUPF_HIP(hipMemcpy2DAsync(m.stage_a.get(), row, grad_va, size_t(grad_va_stride) * sizeof(double),
-                              row, B, hipMemcpyHostToDevice, m.s));
-    CUPF_HIP(hipMemcpy2DAsync(m.stage_b.get(), row, grad_vm, size_t(grad_vm_stride) * sizeof(double),
-                              row, B, hipMemcpyHostToDevice, m.s));
+    m.upload_rows(m.stage_a.get(), grad_va, grad_va_stride, m.n, B, sizeof(double));
+    m.upload_rows(m.stage_b.get(), grad_vm, grad_vm_stride, m.n, B, sizeof(double));
     kern::adjoint_gather<double>(m.nr, B, m.Bp, m.stage_a.as<double>(), m.n,
                                  m.stage_b.as<double>(), m.n, m.g.as<double>(), m.s);
     const auto ts = std::chrono::steady_clock::now();
@@ -1118,14 +1126,10 @@ void NewtonSolver::solve_adjoint(const double* grad_va, int64_t grad_va_stride,
     result.n_bus = m.n;
     result.batch_size = B;
     result.dimF = m.js.dim;
-    {
-        std::vector<double> li(size_t(m.js.dim) * m.Bp);
-        CUPF_HIP(hipMemcpyAsync(li.data(), m.lam.get(), li.size() * sizeof(double),
-                                hipMemcpyDeviceToHost, m.s));
-        CUPF_HIP(hipStreamSynchronize(m.s));
-        result.lambda.resize(size_t(B) * m.js.dim);
-        host_deinterleave(li, B, m.Bp, m.js.dim, result.lambda.data());
-    }
+    kern::from_interleaved(m.lam.as<double>(), m.js.dim, B, m.Bp, m.stage_c.as<double>(), m.js.dim, m.s);
+    result.lambda.resize(size_t(B) * m.js.dim);
+    CUPF_HIP(hipMemcpyAsync(result.lambda.data(), m.stage_c.get(), result.lambda.size() * sizeof(double),
+                            hipMemcpyDeviceToHost, m.s));
     if (options.compute_load_gradients) {
         kern::adjoint_project<double>(m.nr, B, m.Bp, m.lam.as<double>(), m.stage_a.as<double>(),
                                       m.stage_b.as<double>(), m.s);
@@ -1139,19 +1143,19 @@ void NewtonSolver::solve_adjoint(const double* grad_va, int64_t grad_va_stride,
     if (options.check_residual) {
         m.lu.residual<double>(m.J.as<double>(), m.g.as<double>(), m.lam.as<double>(), m.lu.res(),
                               true, m.Bp, m.s);
-        std::vector<double> r(size_t(m.js.dim) * m.Bp), gh(size_t(m.js.dim) * m.Bp);
-        CUPF_HIP(hipMemcpyAsync(r.data(), m.lu.res(), r.size() * sizeof(double),
-                                hipMemcpyDeviceToHost, m.s));
-        CUPF_HIP(hipMemcpyAsync(gh.data(), m.g.get(), gh.size() * sizeof(double),
+        // sums of squares per block of rows on the device, their total here
+        const int parts = kern::sum_squares_parts(m.js.dim, m.Bp);
+        std::vector<double> sums(2 * size_t(parts));
+        kern::sum_squares(m.lu.res(), m.js.dim, B, m.Bp, m.stage_c.as<double>(), m.s);
+        kern::sum_squares(m.g.as<double>(), m.js.dim, B, m.Bp, m.stage_c.as<double>() + parts, m.s);
+        CUPF_HIP(hipMemcpyAsync(sums.data(), m.stage_c.get(), sums.size() * sizeof(double),
                                 hipMemcpyDeviceToHost, m.s));
         CUPF_HIP(hipStreamSynchronize(m.s));
         long double rr = 0, gg = 0;
-        for (int i = 0; i < m.js.dim; ++i)
-            for (int b = 0; b < B; ++b) {
-                const size_t o = size_t(i) * m.Bp + b;
-                rr += (long double)r[o] * r[o];
-                gg += (long double)gh[o] * gh[o];
-            }
+        for (int i = 0; i < parts; ++i) {
+            rr += sums[size_t(i)];
+            gg += sums[size_t(parts + i)];
+        }
         const long double den =
             std::max(std::sqrt(std::max(gg, (long double)1e-60)), (long double)1e-30);
         result.jt_residual_norm = double(std::sqrt(rr) / den);

@@ -302,6 +302,28 @@ __global__ __launch_bounds__(kBlock) void k_axpy(const TX* __restrict__ a, TX* _
     if (i < count) x[i] += a[i];
 }
 
+// Bound by the read of v; a block sums kSumRows rows of 64 scenarios.
+constexpr int kSumRows = 64;
+__global__ __launch_bounds__(kBlock) void k_sum_squares(const double* __restrict__ v, int dim, int B,
+                                                        int Bp, double* __restrict__ out) {
+    const int lane = threadIdx.x & (kLanes - 1), w = threadIdx.x / kLanes;
+    const int b = blockIdx.y * kLanes + lane;
+    double acc = 0.0;
+    if (b < B)
+        for (int i = blockIdx.x * kSumRows + w; i < min(dim, int(blockIdx.x + 1) * kSumRows); i += kWaves) {
+            const double x = v[(long long)i * Bp + b];
+            acc = fma(x, x, acc);
+        }
+    __shared__ double red[kBlock];
+    red[threadIdx.x] = acc;
+    __syncthreads();
+    for (int s = kBlock / 2; s > 0; s >>= 1) {
+        if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) out[blockIdx.y * gridDim.x + blockIdx.x] = red[0];
+}
+
 __global__ __launch_bounds__(kBlock) void k_batch_max(const double* __restrict__ v, int B,
                                                       double* __restrict__ out,
                                                       const int* __restrict__ gate) {
@@ -563,6 +585,14 @@ void axpy_update(const TX* ddx, TX* dx, long long count, hipStream_t s, const in
     const long long blocks = (count + kBlock - 1) / kBlock;
     hipLaunchKernelGGL(k_axpy<TX>, dim3((unsigned)blocks), dim3(kBlock), 0, s, ddx, dx, count,
                        gate);
+    CUPF_HIP(hipGetLastError());
+}
+
+int sum_squares_parts(int dim, int Bp) { return (dim + kSumRows - 1) / kSumRows * (Bp / kLanes); }
+
+void sum_squares(const double* v, int dim, int B, int Bp, double* out, hipStream_t s) {
+    const dim3 grid((dim + kSumRows - 1) / kSumRows, Bp / kLanes);
+    hipLaunchKernelGGL(k_sum_squares, grid, dim3(kBlock), 0, s, v, dim, B, Bp, out);
     CUPF_HIP(hipGetLastError());
 }
 
