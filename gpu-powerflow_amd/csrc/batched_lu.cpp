@@ -309,6 +309,12 @@ void BatchedLU::find_sys(int n_bus, const int* rp, const int* ci, const std::vec
 }
 
 
+int BatchedLU::scenarios(int Bp) const {
+    if (B_ < 1 || B_ > Bp || B_ <= Bp - kern::kLanes)
+        throw std::runtime_error("BatchedLU: set_batch() does not match the padded batch");
+    return B_;
+}
+
 // Chains of nested fronts (FP32 fronts; kern::chain_factor, nested_chains).
 // F0's own level is factored as usual, its pivot + Schur group writing the
 // contribution block to its trailing block.  The additions of each member
@@ -679,6 +685,7 @@ void BatchedLU::factor(const double* A, int Bp, hipStream_t s, StageTimer* timer
                                     opt_.pivot_eps, sp, mem_.sing, sys_lds_, s);
         return;
     }
+    lu_.nb = scenarios(Bp);
     if (opt_.front64) factor_t<double>(A, Bp, s, timer, stage);
     else factor_t<float>(A, Bp, s, timer, stage);
 }
@@ -726,6 +733,7 @@ void BatchedLU::solve_dispatch(const double* rhs, TX* x, bool transpose, int Bp,
                                        B_, Bp, x, transpose, sys_lds_, s);
         return;
     }
+    lu_.nb = scenarios(Bp);
     if (opt_.front64) solve_once<double, TX>(rhs, x, transpose, Bp, s);
     else solve_once<float, TX>(rhs, x, transpose, Bp, s);
 }

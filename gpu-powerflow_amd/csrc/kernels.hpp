@@ -138,6 +138,8 @@ constexpr int kSchurTileCols = 64;
 
 struct LuDevice {
     int n = 0, nnz = 0, P = 0;
+    int nb = 0;                       // real scenarios: the workgroup-per-scenario launches cover
+                                      // these, the lane-per-scenario ones the padded batch
     long long arena0 = 0, arena1 = 0, upd_total = 0;
     const int* fsz = nullptr;
     const int* nc = nullptr;

@@ -30,7 +30,9 @@
 // scenario (or a small group of scenarios) fastest: neighbouring workgroups
 // take neighbouring scenarios, which share the cache lines of the interleaved
 // arrays.  (A remap giving each of the 8 XCDs a contiguous range of the grid
-// measured 5-6 % slower on the factorisation and 3-5 % on the solve.)
+// measured 5-6 % slower on the factorisation and 3-5 % on the solve.)  They
+// cover the real scenarios only; the tier-0 kernels' lanes past them work on
+// whatever the padding holds, and nothing reads what they write.
 #include "kernels.hpp"
 #include "hip_common.hpp"
 
@@ -60,10 +62,10 @@ __device__ inline T guard_pivot(T piv, double eps, int static_piv, int& flag) {
 }
 
 // Flat block id -> (front index in the group, scenario); see file comment.
-__device__ inline void decode_block(int Bp, int& fi, int& b) {
-    const long long w = blockIdx.x;                      // gridDim.x = count * Bp
-    fi = int(w / Bp);
-    b = int(w % Bp);
+__device__ inline void decode_block(int nb, int& fi, int& b) {
+    const long long w = blockIdx.x;                      // gridDim.x = count * nb
+    fi = int(w / nb);
+    b = int(w % nb);
 }
 
 // Pointer to element 0 of front c's contribution-block source for scenario b
@@ -343,7 +345,7 @@ __global__ __launch_bounds__(NT) void k_factor_t1(LuDevice d,
     extern __shared__ unsigned char smem_raw[];
     T* F = reinterpret_cast<T*>(smem_raw);
     int fi, b;
-    decode_block(Bp, fi, b);
+    decode_block(d.nb, fi, b);
     const int p = fronts[fi];
     const int fs = d.fsz[p], ncp = d.nc[p];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -465,7 +467,7 @@ __global__ __launch_bounds__(kFactorBlock) void k_factor_t2(LuDevice d,
     __shared__ T P[kLdsT];
     __shared__ T stage[kKb * kTile];
     int fi, b;
-    decode_block(Bp, fi, b);
+    decode_block(d.nb, fi, b);
     const int p = fronts[fi];
     const int fs = d.fsz[p], ncp = d.nc[p];
     const int tid = threadIdx.x;
@@ -600,8 +602,8 @@ __global__ __launch_bounds__(kAsmThreads) void k_assemble_rows(LuDevice d,
     T* F = reinterpret_cast<T*>(smem_raw);   // [rb_rows][fs]
     // lin -> (front, row block, scenario), scenario fastest
     const long long w = blockIdx.x;
-    const int b = int(w % Bp);
-    const long long rest = w / Bp;
+    const int b = int(w % d.nb);
+    const long long rest = w / d.nb;
     const int rb = int(rest % nrb);
     const int fi = int(rest / nrb);
     const int p = fronts[fi];
@@ -774,7 +776,7 @@ __global__ __launch_bounds__(kDenseThreads) void k_factor_t2_mfma(LuDevice d,
     float* stage = P + size_t(kDenseMaxFsz) * kPld;               // [kDenseKb][kSld]
     float* prow = stage + size_t(kDenseKb) * kSld;                // [2][kDenseKb]
     int fi, b;
-    decode_block(Bp, fi, b);
+    decode_block(d.nb, fi, b);
     const int p = fronts[fi];
     const int fs = d.fsz[p], ncp = d.nc[p];
     const int tid = threadIdx.x;
@@ -1073,7 +1075,7 @@ __global__ __launch_bounds__(pivot_threads<T>()) void k_pivot(LuDevice d, const 
     extern __shared__ unsigned char smem_raw[];
     T* P = reinterpret_cast<T*>(smem_raw);                         // A11: [64][kPivLd], then transposed
     int fi, b;
-    decode_block(Bp, fi, b);
+    decode_block(d.nb, fi, b);
     const int p = fronts[fi];
     const int fs = d.fsz[p], K = d.nc[p];
     constexpr int NT = pivot_threads<T>();
@@ -1325,13 +1327,13 @@ __global__ __launch_bounds__(kSchurThreads, 3) void k_schur(LuDevice d, const in
     w /= kSchurScen;
     const int rb = int(w % nrb);
     w /= nrb;
-    const int ngrp = Bp / kSchurScen;
+    const int ngrp = (d.nb + kSchurScen - 1) / kSchurScen;
     const int b = int(w % ngrp) * kSchurScen + bl;
     const int fi = int(w / ngrp);
     const int p = fronts[fi];
     const int fs = d.fsz[p], K = d.nc[p], uc = fs - K;
     const int i0 = K + rb * RB;
-    if (i0 >= fs) return;                       // whole block exits together
+    if (i0 >= fs || b >= d.nb) return;          // whole block exits together
     const int i1 = min(fs, i0 + RB);
     const int nr = i1 - i0;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1575,7 +1577,7 @@ __global__ __launch_bounds__(kPivThreads) void k_chain_u12(LuDevice d, ChainDevi
     const int p = ch.fronts[k];
     const int fs = d.fsz[p], K = d.nc[p];
     const int j0 = K + chn * kXChunk;
-    if (j0 >= fs || b >= Bp) return;            // whole block exits together
+    if (j0 >= fs || b >= d.nb) return;            // whole block exits together
     const int tid = threadIdx.x;
     float* arena = ar.a1 + (long long)b * d.arena1;
     int ldT;
@@ -1600,7 +1602,7 @@ __global__ __launch_bounds__(kChainThreads, 2) void k_chain_strips(LuDevice d, C
     float* Us = reinterpret_cast<float*>(smem_raw);               // U11^-1 [64][kLinvLd]
     int g, b;
     decode_chain(ngrp, g, b);
-    if (b >= Bp) return;                        // whole block exits together
+    if (b >= d.nb) return;                      // whole block exits together
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     float* Lw = Us + 64 * kLinvLd + wave * kChainStrip * kChainLd;  // this wave's strip
     const int p = ch.fronts[k];
@@ -1848,10 +1850,10 @@ __device__ __forceinline__ void l21_block(const LuDevice& d, const int* __restri
 
 // Block decode of the pivot-row chunk and pivot-column block launches:
 // lin -> (front, part, scenario), scenario fastest.
-__device__ inline void decode_part(int Bp, int parts, int& fi, int& part, int& b) {
+__device__ inline void decode_part(int nb, int parts, int& fi, int& part, int& b) {
     long long w = blockIdx.x;
-    b = int(w % Bp);
-    w /= Bp;
+    b = int(w % nb);
+    w /= nb;
     part = int(w % parts);
     fi = int(w / parts);
 }
@@ -1862,7 +1864,7 @@ __global__ __launch_bounds__(kPivThreads) void k_u12(LuDevice d, const int* __re
                                                       Arenas<T> ar, const T* __restrict__ side,
                                                       int nch) {
     int fi, ch, b;
-    decode_part(Bp, nch, fi, ch, b);
+    decode_part(d.nb, nch, fi, ch, b);
     u12_chunk<T>(d, fronts, A, Bp, ar, side, fi, ch, b);
 }
 
@@ -1871,7 +1873,7 @@ __global__ __launch_bounds__(256) void k_l21(LuDevice d, const int* __restrict__
                                              const double* __restrict__ A, int Bp, Arenas<T> ar,
                                              const T* __restrict__ uinv, int nblk) {
     int fi, blk, b;
-    decode_part(Bp, nblk, fi, blk, b);
+    decode_part(d.nb, nblk, fi, blk, b);
     l21_block<T>(d, fronts, A, Bp, ar, uinv, fi, blk, b);
 }
 
@@ -1888,6 +1890,7 @@ __global__ __launch_bounds__(256, 3) void k_schur_tile(LuDevice d, const int* __
     w /= scen_group;
     const int t = int(w % ntiles);
     const int b = int(w / ntiles) * scen_group + bl;
+    if (b >= d.nb) return;                                       // whole block exits together
     const int2 tl = tiles[t];
     const int p = fronts[tl.x];
     const int rb = tl.y >> 16, ct = tl.y & 0xffff;
@@ -2299,7 +2302,7 @@ __global__ __launch_bounds__(kLanes) void k_fwd_t12(LuDevice d, const int* __res
     T* w = reinterpret_cast<T*>(smem_raw);
     const int lane = threadIdx.x;
     int fi, b;
-    decode_block(Bp, fi, b);
+    decode_block(d.nb, fi, b);
     const int p = fronts[fi];
     const int fs = d.fsz[p], ncp = d.nc[p], uc = fs - ncp;
     const int* fr = d.front_rows + d.front_ptr[p];
@@ -2320,7 +2323,7 @@ __global__ __launch_bounds__(kLanes) void k_bwd_t12(LuDevice d, const int* __res
     T* w = reinterpret_cast<T*>(smem_raw);
     const int lane = threadIdx.x;
     int fi, b;
-    decode_block(Bp, fi, b);
+    decode_block(d.nb, fi, b);
     const int p = fronts[fi];
     const int fs = d.fsz[p], ncp = d.nc[p];
     const int* fr = d.front_rows + d.front_ptr[p];
@@ -2421,7 +2424,7 @@ __global__ __launch_bounds__(NT) void k_fwd_w(LuDevice d, const int* __restrict_
     T* w = P + KM * PLD;                                   // [fs]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int fi, b;
-    decode_block(Bp, fi, b);
+    decode_block(d.nb, fi, b);
     const int p = fronts[fi];
     const int fs = d.fsz[p], K = d.nc[p], uc = fs - K;
     const int* fr = d.front_rows + d.front_ptr[p];
@@ -2477,7 +2480,7 @@ __global__ __launch_bounds__(NT) void k_bwd_w(LuDevice d, const int* __restrict_
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     constexpr int NW = NT / 64;
     int fi, b;
-    decode_block(Bp, fi, b);
+    decode_block(d.nb, fi, b);
     const int p = fronts[fi];
     const int fs = d.fsz[p], K = d.nc[p], uc = fs - K;
     const int* fr = d.front_rows + d.front_ptr[p];
@@ -2573,7 +2576,7 @@ void assemble_rows(const LuDevice& d, const int* fronts, int count, int max_fsz,
     const size_t shmem = size_t(rb_rows) * max_fsz * sizeof(T);
     if (shmem > size_t(kLdsBytes)) throw std::runtime_error("assemble_rows: front row exceeds LDS");
     const int nrb = (max_fsz + rb_rows - 1) / rb_rows;
-    const long long blocks = (long long)count * nrb * Bp;
+    const long long blocks = (long long)count * nrb * d.nb;
     if (blocks >= (1LL << 31)) throw std::runtime_error("assemble_rows: grid too large");
     hipLaunchKernelGGL(k_assemble_rows<T>, dim3(unsigned(blocks)), dim3(kAsmThreads), shmem, s, d,
                        fronts, A, Bp, ar, nrb, rb_rows);
@@ -2600,19 +2603,19 @@ void cross_group(const LuDevice& d, const int* fronts, int count, int max_fsz, c
                                      int(u12_lds<T>())));
         attr_set = true;
     }
-    hipLaunchKernelGGL(k_pivot<T>, dim3(unsigned(count) * unsigned(Bp)), dim3(pivot_threads<T>()),
+    hipLaunchKernelGGL(k_pivot<T>, dim3(unsigned(count) * unsigned(d.nb)), dim3(pivot_threads<T>()),
                        pivot_lds<T>(), s, d,
                        fronts, A, Bp, ar, uinv, pivot_eps, static_piv, sing);
     CUPF_HIP(hipGetLastError());
     const int nch = (max_fsz + kXChunk - 1) / kXChunk;
-    const long long blocks = (long long)count * nch * Bp;
+    const long long blocks = (long long)count * nch * d.nb;
     if (blocks >= (1LL << 31)) throw std::runtime_error("cross_group: grid too large");
     hipLaunchKernelGGL(k_u12<T>, dim3(static_cast<unsigned>(blocks)), dim3(kPivThreads), u12_lds<T>(),
                        s, d, fronts, A, Bp, ar, uinv, nch);
     CUPF_HIP(hipGetLastError());
     if (with_l21) {
         const int nblk = (max_fsz + kL21Rows - 1) / kL21Rows;
-        const long long lb = (long long)count * nblk * Bp;
+        const long long lb = (long long)count * nblk * d.nb;
         if (lb >= (1LL << 31)) throw std::runtime_error("cross_group: grid too large");
         hipLaunchKernelGGL(k_l21<T>, dim3(static_cast<unsigned>(lb)), dim3(256),
                            l21_lds_elems() * sizeof(T), s, d, fronts, A, Bp, ar, uinv, nblk);
@@ -2628,7 +2631,8 @@ void schur_group(const LuDevice& d, const int* fronts, int count, int max_nc, in
     if (max_uc > kDenseMaxFsz || max_nc > kXMaxK || Bp % kSchurScen)
         throw std::runtime_error("schur_group: front or batch outside the kernel's limits");
     const int nrb = (max_uc + schur_rows<T>() - 1) / schur_rows<T>();
-    const long long blocks = (long long)count * nrb * Bp;
+    const long long blocks =
+        (long long)count * nrb * ((d.nb + kSchurScen - 1) / kSchurScen * kSchurScen);
     if (blocks >= (1LL << 31)) throw std::runtime_error("schur_group: grid too large");
     const int sld = schur_ld(max_nc);
     const size_t shmem = schur_lds<T>(sld, max_uc);
@@ -2670,7 +2674,7 @@ void schur_tile_group(const LuDevice& d, const int* fronts, const int2* tiles, i
     if (ntiles <= 0) return;
     if (scen_group < 1 || Bp % scen_group || kLanes % scen_group)
         throw std::runtime_error("schur_tile_group: scenario group must divide 64");
-    const long long blocks = (long long)ntiles * Bp;
+    const long long blocks = (long long)ntiles * ((d.nb + scen_group - 1) / scen_group * scen_group);
     if (blocks >= (1LL << 31)) throw std::runtime_error("schur_tile_group: grid too large");
     const dim3 grid(static_cast<unsigned>(blocks));
     if constexpr (sizeof(T) == 8) {
@@ -2710,22 +2714,22 @@ void chain_factor(const LuDevice& d, const ChainDevice& c, const std::vector<int
         const int fs = fsz[size_t(k)], K = nc[size_t(k)], uc = fs - K;
         if (K < 1 || K > kXMaxK || uc < 0 || o + fs > fsz[0] - nc[0])
             throw std::invalid_argument("chain_factor: front outside the chain's trailing block");
-        hipLaunchKernelGGL(k_chain_pivot, dim3(unsigned(Bp)), dim3(kChainThreads), piv_lds, s, d, c, k, o,
+        hipLaunchKernelGGL(k_chain_pivot, dim3(unsigned(d.nb)), dim3(kChainThreads), piv_lds, s, d, c, k, o,
                            A, Bp, ar, side, pivot_eps, static_piv, sing);
         CUPF_HIP(hipGetLastError());
         if (uc > 0) {
             const int nch = (uc + kXChunk - 1) / kXChunk;
-            hipLaunchKernelGGL(k_chain_u12, dim3(unsigned(nch) * unsigned(Bp)), dim3(kPivThreads), u12_bytes, s,
+            hipLaunchKernelGGL(k_chain_u12, dim3(unsigned(nch) * unsigned(d.nb)), dim3(kPivThreads), u12_bytes, s,
                                d, c, k, o, Bp, ar, side, nch);
             CUPF_HIP(hipGetLastError());
             const int nstrip = (uc + kChainStrip - 1) / kChainStrip;
             const int ngrp = (nstrip + kChainStrips - 1) / kChainStrips;
             const int last = k == c.steps ? 1 : 0;
             if (dense_mode == kMfmaBf16x3)
-                hipLaunchKernelGGL(k_chain_strips<kMfmaBf16x3>, dim3(unsigned(ngrp) * unsigned(Bp)),
+                hipLaunchKernelGGL(k_chain_strips<kMfmaBf16x3>, dim3(unsigned(ngrp) * unsigned(d.nb)),
                                    dim3(kChainThreads), strip_lds, s, d, c, k, o, Bp, ar, side, ngrp, last);
             else
-                hipLaunchKernelGGL(k_chain_strips<kMfmaF32>, dim3(unsigned(ngrp) * unsigned(Bp)),
+                hipLaunchKernelGGL(k_chain_strips<kMfmaF32>, dim3(unsigned(ngrp) * unsigned(d.nb)),
                                    dim3(kChainThreads), strip_lds, s, d, c, k, o, Bp, ar, side, ngrp, last);
             CUPF_HIP(hipGetLastError());
         }
@@ -2754,7 +2758,7 @@ void lu_factor_group(const LuDevice& d, int tier, const int* fronts, int count, 
             attr_set = true;
         }
         Arenas<float> af{reinterpret_cast<float*>(ar.a0), reinterpret_cast<float*>(ar.a1)};
-        const dim3 grid(unsigned(count) * unsigned(Bp));
+        const dim3 grid(unsigned(count) * unsigned(d.nb));
         if (dense_mode == kMfmaBf16x3)
             hipLaunchKernelGGL(k_factor_t2_mfma<kMfmaBf16x3>, grid, dim3(kDenseThreads), kDenseLds, s,
                                d, fronts, A, Bp, af, pivot_eps, static_piv, sing);
@@ -2785,16 +2789,16 @@ void lu_factor_group(const LuDevice& d, int tier, const int* fronts, int count, 
         const size_t shmem = size_t(max_fsz) * max_fsz * sizeof(T);
         if (shmem > size_t(kLdsBytes)) throw std::runtime_error("lu_factor_group: tier-1 front exceeds LDS");
         if (max_fsz <= kT1WaveRows)
-            hipLaunchKernelGGL((k_factor_t1<T, 64>), dim3(unsigned(count) * unsigned(Bp)), dim3(64),
+            hipLaunchKernelGGL((k_factor_t1<T, 64>), dim3(unsigned(count) * unsigned(d.nb)), dim3(64),
                                shmem, s, d, fronts, A, Bp, ar, pivot_eps, static_piv, sing);
         else
-            hipLaunchKernelGGL((k_factor_t1<T, kFactorBlock>), dim3(unsigned(count) * unsigned(Bp)),
+            hipLaunchKernelGGL((k_factor_t1<T, kFactorBlock>), dim3(unsigned(count) * unsigned(d.nb)),
                                dim3(kFactorBlock), shmem, s, d, fronts, A, Bp, ar, pivot_eps,
                                static_piv, sing);
     } else {
         if (max_fsz > kLdsBytes / int(sizeof(T)))
             throw std::runtime_error("lu_factor_group: front exceeds the LDS panel budget");
-        hipLaunchKernelGGL(k_factor_t2<T>, dim3(unsigned(count) * unsigned(Bp)), dim3(kFactorBlock),
+        hipLaunchKernelGGL(k_factor_t2<T>, dim3(unsigned(count) * unsigned(d.nb)), dim3(kFactorBlock),
                            0, s, d, fronts, A, Bp, ar, pivot_eps, static_piv, sing);
     }
     CUPF_HIP(hipGetLastError());
@@ -2805,7 +2809,7 @@ void lu_solve_forward_group(const LuDevice& d, int tier, const int* fronts, int 
                             int max_fsz, int max_nc, Arenas<T> ar, const double* rhs, T* y, T* upd,
                             int Bp, bool transpose, hipStream_t s) {
     if (count <= 0) return;
-    const dim3 grid(unsigned(count) * unsigned(Bp));
+    const dim3 grid(unsigned(count) * unsigned(d.nb));
     if (tier == 0) {
         if (transpose)
             hipLaunchKernelGGL((k_fwd_t0<T, true>), dim3(count, Bp / kLanes), dim3(kLanes), 0, s, d,
@@ -2846,7 +2850,7 @@ void lu_solve_backward_group(const LuDevice& d, int tier, const int* fronts, int
                              int max_fsz, int max_nc, Arenas<T> ar, T* y, int Bp, bool transpose,
                              hipStream_t s) {
     if (count <= 0) return;
-    const dim3 grid(unsigned(count) * unsigned(Bp));
+    const dim3 grid(unsigned(count) * unsigned(d.nb));
     if (tier == 0) {
         if (transpose)
             hipLaunchKernelGGL((k_bwd_t0<T, true>), dim3(count, Bp / kLanes), dim3(kLanes), 0, s, d,
