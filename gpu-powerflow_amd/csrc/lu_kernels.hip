@@ -1919,16 +1919,30 @@ __global__ __launch_bounds__(256, 3) void k_schur_tile(LuDevice d, const int* __
         constexpr int KW = sizeof(T) == 4 ? 32 : 16;             // k run per lane group
         const int g = sizeof(T) == 4 ? lane >> 5 : lane >> 4;
         const int li = sizeof(T) == 4 ? lane & 31 : lane & 15;
-        const bool full = K == kXMaxK;                           // uniform
         const char* Gb = reinterpret_cast<const char*>(G);
         constexpr unsigned ES = unsigned(sizeof(T));
+        // A lane reads a run of its row, 16 bytes a load: a load touches 64
+        // cache lines whatever its width, and element-wide ones (16 per row
+        // run in FP64, 32 in FP32) kept the texture path busy longer than the
+        // update itself.  With 64 columns or more the run stays in the front
+        // (k past K reads elements that are zeroed after the assembly).
+        constexpr int V = 16 / int(sizeof(T));
+        typedef T Run __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+        const bool wide = fs >= kXMaxK;                          // uniform
 #pragma unroll
         for (int s = 0; s < NT; ++s) {
             const int r = min(r0 + 32 * wr + 16 * s + li, fs - 1);
+            if (wide) {
 #pragma unroll
-            for (int i = 0; i < NOP; ++i) {
-                const int k = full ? KW * g + i : min(KW * g + i, K - 1);   // in [0, K)
-                a[s][i] = *reinterpret_cast<const T*>(Gb + unsigned(r * fs + k) * ES);
+                for (int i = 0; i < NOP; i += V) {
+                    const Run run = *reinterpret_cast<const Run*>(Gb + unsigned(r * fs + KW * g + i) * ES);
+#pragma unroll
+                    for (int v = 0; v < V; ++v) a[s][i + v] = run[v];
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < NOP; ++i)
+                    a[s][i] = *reinterpret_cast<const T*>(Gb + unsigned(r * fs + min(KW * g + i, K - 1)) * ES);
             }
         }
     }
