@@ -1878,7 +1878,7 @@ __global__ __launch_bounds__(256) void k_l21(LuDevice d, const int* __restrict__
 }
 
 template <typename T, int MODE>
-__global__ __launch_bounds__(256, 3) void k_schur_tile(LuDevice d, const int* __restrict__ fronts,
+__global__ __launch_bounds__(256, 4) void k_schur_tile(LuDevice d, const int* __restrict__ fronts,
                                                     const int2* __restrict__ tiles, int ntiles,
                                                     int scen_group, const double* __restrict__ A,
                                                     int Bp, Arenas<T> ar) {
@@ -1902,108 +1902,91 @@ __global__ __launch_bounds__(256, 3) void k_schur_tile(LuDevice d, const int* __
     const int wr = wave & 1, wc = wave >> 1;                     // this wave's 32 x 32 quarter
     const bool busy = 32 * wr < nr && 32 * wc < ncl;             // wave-uniform
     T* G = ar.a1 + (long long)b * d.arena1 + d.off[p];
-    const int* rl = d.row_lb + d.lb_ptr[p];
 
-    // ---- L21 operands, in flight during the assembly -------------------------
-    constexpr int NOP = sizeof(T) == 4 ? 32 : 16;
-    constexpr int NT = sizeof(T) == 4 ? 1 : 2;                  // 16 x 16 sub-tiles per side (FP64)
-    T a[NT][NOP], u[NT][NOP];
-    // Rows and columns past the front read its last row / column (the
-    // results there are not stored); pivot indices k at or past K read pivot
-    // column / row K - 1 and are zeroed in the L21 operand after the
-    // assembly.  Every index is clamped into the front (r, c in [0, fs),
-    // k in [0, K)), so all loads are unconditional; the element offsets
-    // r fs + k and k fs + c are below fs^2, and their byte offsets below
-    // 2^32 (fronts are far smaller than 2^29 elements).
-    if (busy) {
-        constexpr int KW = sizeof(T) == 4 ? 32 : 16;             // k run per lane group
-        const int g = sizeof(T) == 4 ? lane >> 5 : lane >> 4;
-        const int li = sizeof(T) == 4 ? lane & 31 : lane & 15;
-        const char* Gb = reinterpret_cast<const char*>(G);
-        constexpr unsigned ES = unsigned(sizeof(T));
-        // A lane reads a run of its row, 16 bytes a load: a load touches 64
-        // cache lines whatever its width, and element-wide ones (16 per row
-        // run in FP64, 32 in FP32) kept the texture path busy longer than the
-        // update itself.  With 64 columns or more the run stays in the front
-        // (k past K reads elements that are zeroed after the assembly).
-        constexpr int V = 16 / int(sizeof(T));
-        typedef T Run __attribute__((ext_vector_type(V), aligned(sizeof(T))));
-        const bool wide = fs >= kXMaxK;                          // uniform
-#pragma unroll
-        for (int s = 0; s < NT; ++s) {
-            const int r = min(r0 + 32 * wr + 16 * s + li, fs - 1);
-            if (wide) {
-#pragma unroll
-                for (int i = 0; i < NOP; i += V) {
-                    const Run run = *reinterpret_cast<const Run*>(Gb + unsigned(r * fs + KW * g + i) * ES);
-#pragma unroll
-                    for (int v = 0; v < V; ++v) a[s][i + v] = run[v];
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < NOP; ++i)
-                    a[s][i] = *reinterpret_cast<const T*>(Gb + unsigned(r * fs + min(KW * g + i, K - 1)) * ES);
-            }
-        }
-    }
-
-    // ---- the tile of A22 ------------------------------------------------------
+    // ---- the tile of A22 (contributions only: the matrix's entries lie in
+    // pivot rows and columns) --------------------------------------------------
     static_assert(tile_lds<T>() % 16 == 0, "16-byte zeroing");
     lds_zero16<256>(At, int(tile_lds<T>() / 16));
-    lds_barrier();
-    put_entries<256>(At, d.ent_dst, d.ent_src, A, Bp, b, rl[r0], rl[r0 + nr], [=](int dst) {
-        const int r = dst / fs, c = dst - r * fs;
-        return (c >= c0 && c < c0 + ncl) ? (r - r0) * LD + c - c0 : -1;
-    });
     lds_barrier();
     assemble_chunks<256, kAsmDepth>(d, ar, d.asm_base[p * kAsmKindCount + kAsmKTile] + rb * nct + ct, b,
                              Bp, At, [=](int rr, int c) { return rr * LD + c - c0; });
     lds_barrier();
     if (!busy) return;                           // no barrier below
-    if (K < kXMaxK) {                            // uniform: k >= K terms of the L21 operand are 0
-        constexpr int KW = sizeof(T) == 4 ? 32 : 16;
-        const int g = sizeof(T) == 4 ? lane >> 5 : lane >> 4;
+
+    // Operands after the assembly: loads return in order, so issued before it
+    // they would only have delayed its own (FP64 x1,024 95.4 -> 91.9 ms).  The
+    // pivots are dealt to the lane groups in runs of kw, so a front of 22
+    // pivots costs 6 MFMA steps and operand loads and not 16.  A lane reads a
+    // run of its L21 row 16 bytes a load: a load touches 64 cache lines
+    // whatever its width.  Rows and columns past the front read its last row /
+    // column (the results there are not stored); pivot indices at or past K
+    // read pivot row K - 1 of U12 and are zeroed in the L21 operand.  Every
+    // element offset stays below fs^2 and its byte offset below 2^32 (fronts
+    // are far smaller than 2^29 elements).
+    constexpr int V = 16 / int(sizeof(T));
+    typedef T Run __attribute__((ext_vector_type(V), aligned(sizeof(T))));
+    const char* Gb = reinterpret_cast<const char*>(G);
+    constexpr unsigned ES = unsigned(sizeof(T));
+    constexpr int kGroups = sizeof(T) == 4 ? 2 : 4;              // lane groups of an MFMA step
+    constexpr int kStep = sizeof(T) == 8 ? 2 : MODE == kMfmaBf16x3 ? 8 : 4;
+    const int kw = (K + kGroups * kStep - 1) / (kGroups * kStep) * kStep;
+    const bool wide = fs >= kGroups * kw;                        // uniform: runs stay in the row
+    const int q = sizeof(T) == 4 ? lane >> 5 : lane >> 4;
+    const int li = sizeof(T) == 4 ? lane & 31 : lane & 15;
+    const int k0 = kw * q;                                       // this lane's first pivot
+    // V elements of row r from pivot k0 + i on, zero past K
+    auto run_of = [&](int r, int i) {
+        Run v;
+        if (wide) {
+            v = *reinterpret_cast<const Run*>(Gb + unsigned(r * fs + k0 + i) * ES);
+        } else {
 #pragma unroll
-        for (int s = 0; s < NT; ++s)
-#pragma unroll
-            for (int i = 0; i < NOP; ++i)
-                if (KW * g + i >= K) a[s][i] = T(0);
-    }
+            for (int t = 0; t < V; ++t)
+                v[t] = *reinterpret_cast<const T*>(Gb + unsigned(r * fs + min(k0 + i + t, K - 1)) * ES);
+        }
+        return v;
+    };
+    auto u_of = [&](int i, int col) {
+        return *reinterpret_cast<const T*>(Gb + unsigned(min(k0 + i, K - 1) * fs + col) * ES);
+    };
 
     if constexpr (sizeof(T) == 4) {
-        const int h = lane >> 5, li = lane & 31;
-        {
-            const int c = min(c0 + 32 * wc + li, fs - 1);
-            const bool full = K == kXMaxK;
-            const char* Gb = reinterpret_cast<const char*>(G);
+        constexpr int NOP = 32;
+        const int r = min(r0 + 32 * wr + li, fs - 1), c = min(c0 + 32 * wc + li, fs - 1);
+        T a[NOP], u[NOP];
 #pragma unroll
-            for (int i = 0; i < NOP; ++i) {
-                const int k = full ? 32 * h + i : min(32 * h + i, K - 1);
-                u[0][i] = *reinterpret_cast<const T*>(Gb + unsigned(k * fs + c) * 4u);
+        for (int i = 0; i < NOP; i += V) {
+            if (i < kw) {                                // uniform
+                const Run v = run_of(r, i);
+#pragma unroll
+                for (int t = 0; t < V; ++t) {
+                    a[i + t] = v[t];
+                    u[i + t] = u_of(i + t, c);
+                }
             }
         }
         floatx16 acc;
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-            const int rr = 32 * wr + (v >> 2) * 8 + h * 4 + (v & 3);
+            const int rr = 32 * wr + (v >> 2) * 8 + q * 4 + (v & 3);
             acc[v] = At[rr * LD + 32 * wc + li];
         }
         if (MODE == kMfmaF32) {
 #pragma unroll
             for (int i = 0; i < NOP; ++i)
-                if (i < K)                               // uniform
-                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(-a[0][i], u[0][i], acc, 0, 0, 0);
+                if (i < kw)                              // uniform
+                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(k0 + i < K ? -a[i] : T(0), u[i], acc, 0, 0, 0);
         } else {
 #pragma unroll
             for (int j = 0; j < NOP / 8; ++j) {
-                if (8 * j < K) {                         // uniform
+                if (8 * j < kw) {                        // uniform
                     bf16x8 ah, al, bh, blo;
 #pragma unroll
                     for (int t8 = 0; t8 < 8; ++t8) {
                         __bf16 hi, lo;
-                        split_bf16(-a[0][8 * j + t8], hi, lo);
+                        split_bf16(k0 + 8 * j + t8 < K ? -a[8 * j + t8] : T(0), hi, lo);
                         ah[t8] = hi; al[t8] = lo;
-                        split_bf16(u[0][8 * j + t8], hi, lo);
+                        split_bf16(u[8 * j + t8], hi, lo);
                         bh[t8] = hi; blo[t8] = lo;
                     }
                     acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh, acc, 0, 0, 0);
@@ -2016,45 +1999,65 @@ __global__ __launch_bounds__(256, 3) void k_schur_tile(LuDevice d, const int* __
         T* Cw = G + (long long)r0 * fs + c0 + cl;
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-            const int rr = 32 * wr + (v >> 2) * 8 + h * 4 + (v & 3);
+            const int rr = 32 * wr + (v >> 2) * 8 + q * 4 + (v & 3);
             if (rr < nr && cl < ncl) Cw[(long long)rr * fs] = acc[v];
         }
     } else {
-        // one 16-column sub-tile at a time: its U12 operands load, then the
-        // two 16 x 16 row tiles update and store
-        const int q = lane >> 4, li = lane & 15;
-        const char* Gb = reinterpret_cast<const char*>(G);
-        const bool full = K == kXMaxK;                           // uniform
+        // the quarter as 2 x 2 sub-tiles of 16 x 16, eight of a lane's pivots
+        // at a time: both operands of a half load together, 64 registers
+        constexpr int NH = 8;
+        doublex4 acc[2][2];
 #pragma unroll
-        for (int c = 0; c < NT; ++c) {
-            const int col = min(c0 + 32 * wc + 16 * c + li, fs - 1);
-            T uc[NOP];
+        for (int c = 0; c < 2; ++c)
 #pragma unroll
-            for (int i = 0; i < NOP; ++i) {
-                const int k = full ? 16 * q + i : min(16 * q + i, K - 1);   // in [0, K)
-                uc[i] = *reinterpret_cast<const T*>(Gb + unsigned(k * fs + col) * 8u);
+            for (int s = 0; s < 2; ++s)
+#pragma unroll
             }
-            doublex4 acc[NT];
-#pragma unroll
-            for (int s = 0; s < NT; ++s)
-#pragma unroll
                 for (int v = 0; v < 4; ++v)
-                    acc[s][v] = At[(32 * wr + 16 * s + q + 4 * v) * LD + 32 * wc + 16 * c + li];
 #pragma unroll
-            for (int i = 0; i < NOP; ++i) {
-                if (i < K) {                             // uniform
+        for (int s = 0; s < 2; ++s)
 #pragma unroll
-                    for (int s = 0; s < NT; ++s)
-                        acc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(-a[s][i], uc[i], acc[s], 0, 0, 0);
+            for (int v = 0; v < 4; ++v) {
+                const int rr = 32 * wr + 16 * s + q + 4 * v;
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const int cl = 32 * wc + 16 * c + li;
+                    if (rr < nr && cl < ncl) G[(long long)(r0 + rr) * fs + c0 + cl] = acc[c][s][v];
                 }
             }
-            const int cl = 32 * wc + 16 * c + li;
+                    acc[c][s][v] = At[(32 * wr + 16 * s + q + 4 * v) * LD + 32 * wc + 16 * c + li];
 #pragma unroll
-            for (int s = 0; s < NT; ++s)
+        for (int h = 0; h < 2; ++h) {
+            if (NH * h < kw) {                           // uniform
+                T a[2][NH], u[2][NH];
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int rr = 32 * wr + 16 * s + q + 4 * v;
-                    if (rr < nr && cl < ncl) G[(long long)(r0 + rr) * fs + c0 + cl] = acc[s][v];
+                for (int i = 0; i < NH; i += V) {
+                    if (NH * h + i < kw) {               // uniform
+#pragma unroll
+                        for (int s = 0; s < 2; ++s) {
+                            const Run v = run_of(min(r0 + 32 * wr + 16 * s + li, fs - 1), NH * h + i);
+#pragma unroll
+                            for (int t = 0; t < V; ++t) a[s][i + t] = v[t];
+                        }
+#pragma unroll
+                        for (int c = 0; c < 2; ++c)
+#pragma unroll
+                            for (int t = 0; t < V; ++t)
+                                u[c][i + t] = u_of(NH * h + i + t, min(c0 + 32 * wc + 16 * c + li, fs - 1));
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < NH; ++i) {
+                    if (NH * h + i < kw) {               // uniform
+                        const bool in = k0 + NH * h + i < K;
+#pragma unroll
+                        for (int s = 0; s < 2; ++s) {
+                            const T na = in ? -a[s][i] : T(0);
+#pragma unroll
+                            for (int c = 0; c < 2; ++c)
+                                acc[c][s] = __builtin_amdgcn_mfma_f64_16x16x4f64(na, u[c][i], acc[c][s], 0, 0, 0);
+                        }
+                    }
                 }
         }
     }
