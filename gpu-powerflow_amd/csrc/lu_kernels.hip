@@ -37,6 +37,7 @@
 #include "hip_common.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace cupf::kern {
 namespace {
@@ -1231,13 +1232,15 @@ inline size_t schur_lds(int sld, int max_uc) {
 // element t8 of group kq = 16 kq + 8 (lane/32) + t8).  Columns j (< uc) of
 // U12, whose row k starts at U + k * fs; loads from indices clamped into the
 // block, zeroed outside it.
-template <int MODE>
+// KM: the most pivots (32 or 64); operands of absent pivots cost loads and
+// registers all the same.
+template <int MODE, int KM = kXMaxK>
 struct U12Half {
-    float b[kXMaxK / 2];
+    float b[KM / 2];
 };
-template <>
-struct U12Half<kMfmaBf16x3> {
-    bf16x8 h[kXMaxK / 16], l[kXMaxK / 16];
+template <int KM>
+struct U12Half<kMfmaBf16x3, KM> {
+    bf16x8 h[KM / 16], l[KM / 16];
 };
 
 // Load of base[e] by a 32-bit byte offset from a workgroup-uniform base
@@ -1249,14 +1252,14 @@ __device__ __forceinline__ void st_off(float* base, int e, float v) {
     *reinterpret_cast<float*>(reinterpret_cast<char*>(base) + unsigned(e) * 4u) = v;
 }
 
-template <int MODE>
-__device__ __forceinline__ void u12_half_load(U12Half<MODE>& o, const float* __restrict__ U, int j,
+template <int MODE, int KM>
+__device__ __forceinline__ void u12_half_load(U12Half<MODE, KM>& o, const float* __restrict__ U, int j,
                                               int uc, int fs, int K) {
     const int lane = int(threadIdx.x) & 63;
     const bool ok = j < uc;
     const int cj = min(j, uc - 1);
 #pragma unroll
-    for (int i = 0; i < kXMaxK / 2; ++i) {
+    for (int i = 0; i < KM / 2; ++i) {
         const int k = MODE == kMfmaF32 ? 2 * i + (lane >> 5) : 16 * (i >> 3) + 8 * (lane >> 5) + (i & 7);
         const float v = ld_off(U, min(k, K - 1) * fs + cj);
         const float x = (k < K && ok) ? v : 0.f;
@@ -1273,13 +1276,13 @@ __device__ __forceinline__ void u12_half_load(U12Half<MODE>& o, const float* __r
 
 // acc -= L21 U12 over k < K for one 32 x 32 tile with held operands: L21 row
 // lane % 32 at Lrow (LDS).
-template <int MODE>
-__device__ __forceinline__ void cb_half_update(floatx16& acc, const U12Half<MODE>& o,
+template <int MODE, int KM>
+__device__ __forceinline__ void cb_half_update(floatx16& acc, const U12Half<MODE, KM>& o,
                                                const float* __restrict__ Lrow, int K) {
     const int lane = int(threadIdx.x) & 63;
     if constexpr (MODE == kMfmaBf16x3) {
 #pragma unroll
-        for (int kq = 0; kq < kXMaxK / 16; ++kq) {
+        for (int kq = 0; kq < KM / 16; ++kq) {
             if (16 * kq < K) {              // uniform
                 const int kb8 = 16 * kq + 8 * (lane >> 5);
                 bf16x8 ah, al;
@@ -1296,7 +1299,7 @@ __device__ __forceinline__ void cb_half_update(floatx16& acc, const U12Half<MODE
         }
     } else {
 #pragma unroll
-        for (int i = 0; i < kXMaxK / 2; ++i) {
+        for (int i = 0; i < KM / 2; ++i) {
             if (2 * i < K) {                // uniform
                 const float a = -Lrow[2 * i + (lane >> 5)];
                 acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, o.b[i], acc, 0, 0, 0);
@@ -1308,7 +1311,7 @@ __device__ __forceinline__ void cb_half_update(floatx16& acc, const U12Half<MODE
 // Three workgroups per CU: the 32 x 32 update tiles keep the kernel within
 // 168 VGPRs; the LDS (schur_lds) allows three up to 392 contribution columns
 // at <= 32 pivots.
-template <typename T, int MODE>
+template <typename T, int MODE, int KM>
 __global__ __launch_bounds__(kSchurThreads, 3) void k_schur(LuDevice d, const int* __restrict__ fronts,
                                                          const double* __restrict__ A, int Bp,
                                                          Arenas<T> ar,
@@ -1343,13 +1346,13 @@ __global__ __launch_bounds__(kSchurThreads, 3) void k_schur(LuDevice d, const in
 
     // U11^-1 operands of the L21 tiles (waves 0 and 1, MFMA modes), in flight
     // during the assembly: B-operand k = 2 i + lane / 32, column jc
-    float ub[kXMaxK / 2];
+    float ub[KM / 2];
     const int jc = 32 * wave + (lane & 31);              // L21 column of this lane
     const bool l21w = MODE != kMfmaNone && wave < 2 && 32 * wave < K;   // waves forming L21
     if constexpr (MODE != kMfmaNone) {
         if (l21w) {
 #pragma unroll
-            for (int i = 0; i < kXMaxK / 2; ++i) {
+            for (int i = 0; i < KM / 2; ++i) {
                 const int k = 2 * i + (lane >> 5);
                 ub[i] = k < 32 * wave + 32 ? float(Ui[k * kXMaxK + jc]) : 0.f;   // U11^-1 upper
             }
@@ -1420,8 +1423,8 @@ __global__ __launch_bounds__(kSchurThreads, 3) void k_schur(LuDevice d, const in
         // ---- U12 operands (B of the update) of one 32 x 32 tile per wave;
         // the first tile's load while L21 is formed
         const int nt32 = (uc + 31) / 32;
-        U12Half<MODE> ops;
-        if (wave < nt32) u12_half_load<MODE>(ops, G + K, wave * 32 + (lane & 31), uc, fs, K);
+        U12Half<MODE, KM> ops;
+        if (wave < nt32) u12_half_load<MODE, KM>(ops, G + K, wave * 32 + (lane & 31), uc, fs, K);
 
         // ---- L21 = A21 U11^-1 (two 32 x 32 tiles, waves 0 and 1) -----------
         {
@@ -1430,7 +1433,7 @@ __global__ __launch_bounds__(kSchurThreads, 3) void k_schur(LuDevice d, const in
             for (int v = 0; v < 16; ++v) acc[v] = 0.f;
             if (l21w) {                                   // wave-uniform
 #pragma unroll
-                for (int i = 0; i < kXMaxK / 2; ++i) {
+                for (int i = 0; i < KM / 2; ++i) {
                     if (2 * i < 32 * wave + 32) {         // U11^-1 upper: k <= j
                         const float av = Lb[(lane & 31) * sld + 2 * i + (lane >> 5)];
                         acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av, ub[i], acc, 0, 0, 0);
@@ -1460,10 +1463,10 @@ __global__ __launch_bounds__(kSchurThreads, 3) void k_schur(LuDevice d, const in
                 const int rr = (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);
                 acc[v] = oka ? Ab[rr * uc + ja] : 0.f;
             }
-            cb_half_update<MODE>(acc, ops, Lb + (lane & 31) * sld, K);
+            cb_half_update<MODE, KM>(acc, ops, Lb + (lane & 31) * sld, K);
             // next tile's U12 operands in flight during this tile's stores
             if (t + kSchurThreads / 64 < nt32)
-                u12_half_load<MODE>(ops, G + K, ja + 32 * (kSchurThreads / 64), uc, fs, K);
+                u12_half_load<MODE, KM>(ops, G + K, ja + 32 * (kSchurThreads / 64), uc, fs, K);
             float* Cw = G + (long long)i0 * fs + K + ja;
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
@@ -1963,7 +1966,6 @@ __global__ __launch_bounds__(256, 4) void k_schur_tile(LuDevice d, const int* __
                     a[i + t] = v[t];
                     u[i + t] = u_of(i + t, c);
                 }
-            }
         }
         floatx16 acc;
 #pragma unroll
@@ -2010,10 +2012,8 @@ __global__ __launch_bounds__(256, 4) void k_schur_tile(LuDevice d, const int* __
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
-            for (int s = 0; s < 2; ++s)
-#pragma unroll
             }
-                for (int v = 0; v < 4; ++v)
+            for (int s = 0; s < 2; ++s)
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -2025,6 +2025,9 @@ __global__ __launch_bounds__(256, 4) void k_schur_tile(LuDevice d, const int* __
                     if (rr < nr && cl < ncl) G[(long long)(r0 + rr) * fs + c0 + cl] = acc[c][s][v];
                 }
             }
+#pragma unroll
+            }
+                for (int v = 0; v < 4; ++v)
                     acc[c][s][v] = At[(32 * wr + 16 * s + q + 4 * v) * LD + 32 * wc + 16 * c + li];
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -2602,6 +2605,22 @@ void assemble_rows(const LuDevice& d, const int* fronts, int count, int max_fsz,
 
 bool cross_schur_path(int max_fsz, int max_nc) {
     (void)max_fsz;
+// KM: the launch's fronts have at most this many pivots.
+template <typename T, int MODE, int KM>
+void launch_schur(const LuDevice& d, const int* fronts, const double* A, int Bp, Arenas<T> ar, const T* uinv,
+                  int nrb, int sld, unsigned blocks, size_t shmem, hipStream_t s) {
+    static bool attr_set = false;
+    if (!attr_set) {
+        CUPF_HIP(hipFuncSetAttribute((const void*)k_schur<T, MODE, KM>,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     int(schur_lds<T>(kSLd, kDenseMaxFsz))));
+        attr_set = true;
+    }
+    hipLaunchKernelGGL((k_schur<T, MODE, KM>), dim3(blocks), dim3(kSchurThreads), shmem, s, d, fronts, A, Bp,
+                       ar, uinv, nrb, sld);
+    CUPF_HIP(hipGetLastError());
+}
+
     return max_nc <= kXMaxK;
 }
 
@@ -2615,6 +2634,12 @@ void cross_group(const LuDevice& d, const int* fronts, int count, int max_fsz, c
     static bool attr_set = false;
     if (!attr_set) {
         CUPF_HIP(hipFuncSetAttribute((const void*)k_pivot<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    auto go = [&](auto mode, auto most_pivots) {
+        launch_schur<T, decltype(mode)::value, decltype(most_pivots)::value>(
+            d, fronts, A, Bp, ar, uinv, nrb, sld, unsigned(blocks), shmem, s);
+    };
+    using Few = std::integral_constant<int, 32>;
+    using All = std::integral_constant<int, kXMaxK>;
                                      int(pivot_lds<T>())));
         CUPF_HIP(hipFuncSetAttribute((const void*)k_u12<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      int(u12_lds<T>())));
@@ -2623,7 +2648,6 @@ void cross_group(const LuDevice& d, const int* fronts, int count, int max_fsz, c
     hipLaunchKernelGGL(k_pivot<T>, dim3(unsigned(count) * unsigned(d.nb)), dim3(pivot_threads<T>()),
                        pivot_lds<T>(), s, d,
                        fronts, A, Bp, ar, uinv, pivot_eps, static_piv, sing);
-    CUPF_HIP(hipGetLastError());
     const int nch = (max_fsz + kXChunk - 1) / kXChunk;
     const long long blocks = (long long)count * nch * d.nb;
     if (blocks >= (1LL << 31)) throw std::runtime_error("cross_group: grid too large");
@@ -2654,32 +2678,13 @@ void schur_group(const LuDevice& d, const int* fronts, int count, int max_nc, in
     const int sld = schur_ld(max_nc);
     const size_t shmem = schur_lds<T>(sld, max_uc);
     if constexpr (sizeof(T) == 8) {
-        static bool attr_set = false;
-        if (!attr_set) {
-            CUPF_HIP(hipFuncSetAttribute((const void*)k_schur<double, kMfmaNone>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         int(schur_lds<double>(kSLd, kDenseMaxFsz))));
-            attr_set = true;
-        }
-        hipLaunchKernelGGL((k_schur<double, kMfmaNone>), dim3(unsigned(blocks)), dim3(kSchurThreads), shmem,
-                           s, d, fronts, A, Bp, ar, uinv, nrb, sld);
+        go(std::integral_constant<int, kMfmaNone>{}, All{});
+    } else if (dense_mode == kMfmaBf16x3) {
+        if (max_nc <= Few::value) go(std::integral_constant<int, kMfmaBf16x3>{}, Few{});
+        else go(std::integral_constant<int, kMfmaBf16x3>{}, All{});
     } else {
-        static bool attr_set = false;
-        if (!attr_set) {
-            CUPF_HIP(hipFuncSetAttribute((const void*)k_schur<float, kMfmaF32>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         int(schur_lds<float>(kSLd, kDenseMaxFsz))));
-            CUPF_HIP(hipFuncSetAttribute((const void*)k_schur<float, kMfmaBf16x3>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         int(schur_lds<float>(kSLd, kDenseMaxFsz))));
-            attr_set = true;
-        }
-        if (dense_mode == kMfmaBf16x3)
-            hipLaunchKernelGGL((k_schur<float, kMfmaBf16x3>), dim3(unsigned(blocks)), dim3(kSchurThreads),
-                               shmem, s, d, fronts, A, Bp, ar, uinv, nrb, sld);
-        else
-            hipLaunchKernelGGL((k_schur<float, kMfmaF32>), dim3(unsigned(blocks)), dim3(kSchurThreads),
-                               shmem, s, d, fronts, A, Bp, ar, uinv, nrb, sld);
+        if (max_nc <= Few::value) go(std::integral_constant<int, kMfmaF32>{}, Few{});
+        else go(std::integral_constant<int, kMfmaF32>{}, All{});
     }
     CUPF_HIP(hipGetLastError());
 }
