@@ -381,7 +381,7 @@ void BatchedLU::find_chains(hipStream_t s) {
     }
 }
 
-// Tier-1 groups (and FP32 tier-0 groups) are launched in parts of similar LDS
+// Tier-1 and tier-0 groups are launched in parts of similar LDS
 // need: a tier-1 workgroup holds its front in fsz^2 elements of LDS sized by
 // the launch's largest front (a tier-0 workgroup its 64 lanes' fronts), so one
 // launch over fronts of 34 to 128 rows would run every workgroup at the
@@ -396,7 +396,7 @@ void BatchedLU::split_tier1() {
         const double b = double(P.fsz[f]) * P.fsz[f] * double(front_bytes());
         return std::min(8, std::max(1, int(lds_cu / std::max(1.0, b))));
     };
-    // tier 0 (FP32): 64 lanes' fronts of the launch's largest size in LDS per
+    // tier 0: 64 lanes' fronts of the launch's largest size in LDS per
     // workgroup
     auto per_cu0 = [&](int f) {
         const double b = double(P.fsz[f]) * P.fsz[f] * 64.0 * double(front_bytes());
@@ -411,8 +411,7 @@ void BatchedLU::split_tier1() {
         for (int st = g0; st < g1;) {
             const int occ = per_cu0(P.group_fronts[size_t(st)]);
             int en = st + 1;
-            // FP64 tier-0 fronts above 11 rows do not fit the LDS kernel: one launch
-            while (en < g1 && (opt_.front64 || per_cu0(P.group_fronts[size_t(en)]) < 2 * occ)) ++en;
+            while (en < g1 && per_cu0(P.group_fronts[size_t(en)]) < 2 * occ) ++en;
             t0_parts_[size_t(L)].push_back({st - g0, en - st, P.fsz[P.group_fronts[size_t(st)]]});
             st = en;
         }

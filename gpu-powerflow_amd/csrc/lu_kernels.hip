@@ -199,55 +199,17 @@ __device__ __forceinline__ bool gate_closed(const int* gate) { return gate && *g
 // ===========================================================================
 // Factor, tier 0 (lane per scenario)
 // ===========================================================================
-template <typename T>
-__global__ __launch_bounds__(kLanes) void k_factor_t0(LuDevice d, const int* __restrict__ fronts,
-                                                      const double* __restrict__ A, int Bp,
-                                                      Arenas<T> ar, double eps, int static_piv,
-                                                      int* __restrict__ sing) {
-    const int p = fronts[blockIdx.x];
-    const int b = blockIdx.y * kLanes + threadIdx.x;
-    const int fs = d.fsz[p], ncp = d.nc[p];
-    T* G = ar.a0 + d.off[p] * Bp + b;
-    const long long s = Bp;
-    for (int e = 0; e < fs * fs; ++e) G[e * s] = T(0);
-    for (int e = d.ent_ptr[p]; e < d.ent_ptr[p + 1]; ++e)
-        G[d.ent_dst[e] * s] = T(A[(long long)d.ent_src[e] * Bp + b]);
-    for (int q = d.child_ptr[p]; q < d.child_ptr[p + 1]; ++q) {
-        const int c = d.child_idx[q];
-        const int cfs = d.fsz[c], cnc = d.nc[c], cuc = cfs - cnc;
-        long long cs;
-        const T* C = front_ptr(d, ar, c, b, Bp, cs);
-        const int* loc = d.asm_loc + d.asm_ptr[c];
-        for (int a = 0; a < cuc; ++a) {
-            const int ra = loc[a] * fs;
-            const T* crow = C + (long long)((cnc + a) * cfs + cnc) * cs;
-            for (int bb = 0; bb < cuc; ++bb) G[(ra + loc[bb]) * s] += crow[bb * cs];
-        }
-    }
-    int flag = 0;
-    for (int k = 0; k < ncp; ++k) {
-        const T piv = G[(k * fs + k) * s];
-        const T g = guard_pivot(piv, eps, static_piv, flag);
-        if (g != piv) G[(k * fs + k) * s] = g;
-        for (int i = k + 1; i < fs; ++i) {
-            const T l = G[(i * fs + k) * s] / g;
-            G[(i * fs + k) * s] = l;
-            for (int j = k + 1; j < fs; ++j) G[(i * fs + j) * s] -= l * G[(k * fs + j) * s];
-        }
-    }
-    if (flag && !gate_closed(d.gate)) atomicOr(sing + b, 1);
-}
-
-// Tier 0 by four waves over one LDS copy of 64 scenarios' fronts
+// Tier 0 by W waves over one LDS copy of 64 scenarios' fronts
 // (F[e * 64 + lane], lane = scenario): the zeroing, the entries and each
 // child's contribution elements are split over the waves (a child's elements
 // land on distinct positions; children one after another), then at each
 // pivot wave 0 guards the pivot and the rows below are split over the waves,
-// each row with k_factor_t0's arithmetic in its order; last, the factored
-// fronts go to the interleaved arena.  The lane's serial chain of k_factor_t0
-// becomes a quarter as long and waits on LDS instead of global memory.
-template <typename T>
-__global__ __launch_bounds__(256) void k_factor_t0_w4(LuDevice d, const int* __restrict__ fronts,
+// one row a wave at a time; last, the factored fronts go to the interleaved
+// arena.  Bound by the chain of LDS accesses of a wave's rows, and by the one
+// workgroup per CU that a 16-row FP64 front's 128 KiB leave: 16 waves for
+// fronts above kT0WideRows, four for smaller ones.
+template <typename T, int W>
+__global__ __launch_bounds__(64 * W) void k_factor_t0(LuDevice d, const int* __restrict__ fronts,
                                                       const double* __restrict__ A, int Bp,
                                                       Arenas<T> ar, double eps, int static_piv,
                                                       int* __restrict__ sing) {
@@ -257,9 +219,9 @@ __global__ __launch_bounds__(256) void k_factor_t0_w4(LuDevice d, const int* __r
     const int p = fronts[blockIdx.x];
     const int b = blockIdx.y * kLanes + lane;
     const int fs = d.fsz[p], ncp = d.nc[p];
-    for (int e = wave; e < fs * fs; e += 4) F[e * kLanes] = T(0);
+    for (int e = wave; e < fs * fs; e += W) F[e * kLanes] = T(0);
     __syncthreads();
-    for (int e = d.ent_ptr[p] + wave; e < d.ent_ptr[p + 1]; e += 4)
+    for (int e = d.ent_ptr[p] + wave; e < d.ent_ptr[p + 1]; e += W)
         F[d.ent_dst[e] * kLanes] = T(A[(long long)d.ent_src[e] * Bp + b]);
     __syncthreads();
     for (int q = d.child_ptr[p]; q < d.child_ptr[p + 1]; ++q) {
@@ -268,7 +230,7 @@ __global__ __launch_bounds__(256) void k_factor_t0_w4(LuDevice d, const int* __r
         long long cs;
         const T* C = front_ptr(d, ar, c, b, Bp, cs);
         const int* loc = d.asm_loc + d.asm_ptr[c];
-        for (int e = wave; e < cuc * cuc; e += 4) {
+        for (int e = wave; e < cuc * cuc; e += W) {
             const int a = e / cuc, bb = e - a * cuc;
             F[(loc[a] * fs + loc[bb]) * kLanes] += C[(long long)((cnc + a) * cfs + cnc + bb) * cs];
         }
@@ -282,7 +244,7 @@ __global__ __launch_bounds__(256) void k_factor_t0_w4(LuDevice d, const int* __r
         }
         __syncthreads();
         const T g = F[(k * fs + k) * kLanes];
-        for (int i = k + 1 + wave; i < fs; i += 4) {
+        for (int i = k + 1 + wave; i < fs; i += W) {
             const T l = F[(i * fs + k) * kLanes] / g;
             F[(i * fs + k) * kLanes] = l;
             for (int j = k + 1; j < fs; ++j) F[(i * fs + j) * kLanes] -= l * F[(k * fs + j) * kLanes];
@@ -290,7 +252,7 @@ __global__ __launch_bounds__(256) void k_factor_t0_w4(LuDevice d, const int* __r
         __syncthreads();
     }
     T* G = ar.a0 + d.off[p] * Bp + b;
-    for (int e = wave; e < fs * fs; e += 4) G[(long long)e * Bp] = F[e * kLanes];
+    for (int e = wave; e < fs * fs; e += W) G[(long long)e * Bp] = F[e * kLanes];
     if (wave == 0 && flag && !gate_closed(d.gate)) atomicOr(sing + b, 1);
 }
 
@@ -1966,6 +1928,7 @@ __global__ __launch_bounds__(256, 4) void k_schur_tile(LuDevice d, const int* __
                     a[i + t] = v[t];
                     u[i + t] = u_of(i + t, c);
                 }
+            }
         }
         floatx16 acc;
 #pragma unroll
@@ -2012,21 +1975,8 @@ __global__ __launch_bounds__(256, 4) void k_schur_tile(LuDevice d, const int* __
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
-            }
             for (int s = 0; s < 2; ++s)
 #pragma unroll
-        for (int s = 0; s < 2; ++s)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int rr = 32 * wr + 16 * s + q + 4 * v;
-#pragma unroll
-                for (int c = 0; c < 2; ++c) {
-                    const int cl = 32 * wc + 16 * c + li;
-                    if (rr < nr && cl < ncl) G[(long long)(r0 + rr) * fs + c0 + cl] = acc[c][s][v];
-                }
-            }
-#pragma unroll
-            }
                 for (int v = 0; v < 4; ++v)
                     acc[c][s][v] = At[(32 * wr + 16 * s + q + 4 * v) * LD + 32 * wc + 16 * c + li];
 #pragma unroll
@@ -2062,7 +2012,19 @@ __global__ __launch_bounds__(256, 4) void k_schur_tile(LuDevice d, const int* __
                         }
                     }
                 }
+            }
         }
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int rr = 32 * wr + 16 * s + q + 4 * v;
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    const int cl = 32 * wc + 16 * c + li;
+                    if (rr < nr && cl < ncl) G[(long long)(r0 + rr) * fs + c0 + cl] = acc[c][s][v];
+                }
+            }
     }
 }
 
@@ -2605,22 +2567,6 @@ void assemble_rows(const LuDevice& d, const int* fronts, int count, int max_fsz,
 
 bool cross_schur_path(int max_fsz, int max_nc) {
     (void)max_fsz;
-// KM: the launch's fronts have at most this many pivots.
-template <typename T, int MODE, int KM>
-void launch_schur(const LuDevice& d, const int* fronts, const double* A, int Bp, Arenas<T> ar, const T* uinv,
-                  int nrb, int sld, unsigned blocks, size_t shmem, hipStream_t s) {
-    static bool attr_set = false;
-    if (!attr_set) {
-        CUPF_HIP(hipFuncSetAttribute((const void*)k_schur<T, MODE, KM>,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     int(schur_lds<T>(kSLd, kDenseMaxFsz))));
-        attr_set = true;
-    }
-    hipLaunchKernelGGL((k_schur<T, MODE, KM>), dim3(blocks), dim3(kSchurThreads), shmem, s, d, fronts, A, Bp,
-                       ar, uinv, nrb, sld);
-    CUPF_HIP(hipGetLastError());
-}
-
     return max_nc <= kXMaxK;
 }
 
@@ -2634,12 +2580,6 @@ void cross_group(const LuDevice& d, const int* fronts, int count, int max_fsz, c
     static bool attr_set = false;
     if (!attr_set) {
         CUPF_HIP(hipFuncSetAttribute((const void*)k_pivot<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
-    auto go = [&](auto mode, auto most_pivots) {
-        launch_schur<T, decltype(mode)::value, decltype(most_pivots)::value>(
-            d, fronts, A, Bp, ar, uinv, nrb, sld, unsigned(blocks), shmem, s);
-    };
-    using Few = std::integral_constant<int, 32>;
-    using All = std::integral_constant<int, kXMaxK>;
                                      int(pivot_lds<T>())));
         CUPF_HIP(hipFuncSetAttribute((const void*)k_u12<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                      int(u12_lds<T>())));
@@ -2648,6 +2588,7 @@ void cross_group(const LuDevice& d, const int* fronts, int count, int max_fsz, c
     hipLaunchKernelGGL(k_pivot<T>, dim3(unsigned(count) * unsigned(d.nb)), dim3(pivot_threads<T>()),
                        pivot_lds<T>(), s, d,
                        fronts, A, Bp, ar, uinv, pivot_eps, static_piv, sing);
+    CUPF_HIP(hipGetLastError());
     const int nch = (max_fsz + kXChunk - 1) / kXChunk;
     const long long blocks = (long long)count * nch * d.nb;
     if (blocks >= (1LL << 31)) throw std::runtime_error("cross_group: grid too large");
@@ -2664,6 +2605,22 @@ void cross_group(const LuDevice& d, const int* fronts, int count, int max_fsz, c
     }
 }
 
+// KM: the launch's fronts have at most this many pivots.
+template <typename T, int MODE, int KM>
+void launch_schur(const LuDevice& d, const int* fronts, const double* A, int Bp, Arenas<T> ar, const T* uinv,
+                  int nrb, int sld, unsigned blocks, size_t shmem, hipStream_t s) {
+    static bool attr_set = false;
+    if (!attr_set) {
+        CUPF_HIP(hipFuncSetAttribute((const void*)k_schur<T, MODE, KM>,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize,
+                                     int(schur_lds<T>(kSLd, kDenseMaxFsz))));
+        attr_set = true;
+    }
+    hipLaunchKernelGGL((k_schur<T, MODE, KM>), dim3(blocks), dim3(kSchurThreads), shmem, s, d, fronts, A, Bp,
+                       ar, uinv, nrb, sld);
+    CUPF_HIP(hipGetLastError());
+}
+
 template <typename T>
 void schur_group(const LuDevice& d, const int* fronts, int count, int max_nc, int max_uc,
                  const double* A, int Bp, Arenas<T> ar, const T* uinv, int dense_mode,
@@ -2677,6 +2634,12 @@ void schur_group(const LuDevice& d, const int* fronts, int count, int max_nc, in
     if (blocks >= (1LL << 31)) throw std::runtime_error("schur_group: grid too large");
     const int sld = schur_ld(max_nc);
     const size_t shmem = schur_lds<T>(sld, max_uc);
+    auto go = [&](auto mode, auto most_pivots) {
+        launch_schur<T, decltype(mode)::value, decltype(most_pivots)::value>(
+            d, fronts, A, Bp, ar, uinv, nrb, sld, unsigned(blocks), shmem, s);
+    };
+    using Few = std::integral_constant<int, 32>;
+    using All = std::integral_constant<int, kXMaxK>;
     if constexpr (sizeof(T) == 8) {
         go(std::integral_constant<int, kMfmaNone>{}, All{});
     } else if (dense_mode == kMfmaBf16x3) {
@@ -2686,7 +2649,6 @@ void schur_group(const LuDevice& d, const int* fronts, int count, int max_nc, in
         if (max_nc <= Few::value) go(std::integral_constant<int, kMfmaF32>{}, Few{});
         else go(std::integral_constant<int, kMfmaF32>{}, All{});
     }
-    CUPF_HIP(hipGetLastError());
 }
 
 template <typename T>
@@ -2763,6 +2725,25 @@ size_t pivot_side_elems(int count, int Bp) { return size_t(count) * Bp * kSideEl
 
 int schur_block_rows(int elem) { return elem == 4 ? schur_rows<float>() : schur_rows<double>(); }
 
+// Fronts above this many rows take 16 waves.
+constexpr int kT0WideRows = 8;
+
+template <typename T, int W>
+void launch_t0(const LuDevice& d, const int* fronts, int count, int max_fsz, const double* A, int Bp,
+               Arenas<T> ar, double pivot_eps, int static_piv, int* sing, hipStream_t s) {
+    constexpr size_t most = size_t(kTier0Max) * kTier0Max * kLanes * sizeof(T);
+    static_assert(most <= 160 * 1024, "a tier-0 front of 64 scenarios in LDS");
+    static bool attr_set = false;
+    if (!attr_set) {
+        CUPF_HIP(hipFuncSetAttribute((const void*)k_factor_t0<T, W>,
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(most)));
+        attr_set = true;
+    }
+    const size_t shmem = size_t(max_fsz) * max_fsz * kLanes * sizeof(T);
+    hipLaunchKernelGGL((k_factor_t0<T, W>), dim3(count, Bp / kLanes), dim3(64 * W), shmem, s, d, fronts, A, Bp,
+                       ar, pivot_eps, static_piv, sing);
+}
+
 template <typename T>
 void lu_factor_group(const LuDevice& d, int tier, const int* fronts, int count, int max_fsz,
                      const double* A, int Bp, Arenas<T> ar, double pivot_eps, int static_piv,
@@ -2793,20 +2774,8 @@ void lu_factor_group(const LuDevice& d, int tier, const int* fronts, int count, 
     }
     if (tier == 0) {
         if (max_fsz > kTier0Max) throw std::runtime_error("lu_factor_group: tier-0 front too large");
-        const size_t shmem = size_t(max_fsz) * max_fsz * kLanes * sizeof(T);
-        if (shmem <= size_t(kLdsBytes)) {
-            static bool attr_set = false;
-            if (!attr_set) {
-                CUPF_HIP(hipFuncSetAttribute((const void*)k_factor_t0_w4<T>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));
-                attr_set = true;
-            }
-            hipLaunchKernelGGL(k_factor_t0_w4<T>, dim3(count, Bp / kLanes), dim3(256), shmem, s, d, fronts,
-                               A, Bp, ar, pivot_eps, static_piv, sing);
-        } else {
-            hipLaunchKernelGGL(k_factor_t0<T>, dim3(count, Bp / kLanes), dim3(kLanes), 0, s, d, fronts,
-                               A, Bp, ar, pivot_eps, static_piv, sing);
-        }
+        if (max_fsz > kT0WideRows) launch_t0<T, 16>(d, fronts, count, max_fsz, A, Bp, ar, pivot_eps, static_piv, sing, s);
+        else launch_t0<T, 4>(d, fronts, count, max_fsz, A, Bp, ar, pivot_eps, static_piv, sing, s);
     } else if (tier == 1) {
         const size_t shmem = size_t(max_fsz) * max_fsz * sizeof(T);
         if (shmem > size_t(kLdsBytes)) throw std::runtime_error("lu_factor_group: tier-1 front exceeds LDS");
