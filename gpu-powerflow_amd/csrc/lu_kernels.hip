@@ -928,7 +928,7 @@ constexpr size_t pivot_lds() {
 
 template <typename T>
 constexpr size_t u12_lds() {
-    return size_t(64 * kLinvLd + 64 * kXCld) * sizeof(T);
+    return size_t(64 * kXCld) * sizeof(T);
 }
 
 // Pivot block of one (front, scenario), four waves (two also work: the
@@ -1061,27 +1061,57 @@ __global__ __launch_bounds__(pivot_threads<T>()) void k_pivot(LuDevice d, const 
                         sing + b, d.gate);
 }
 
+// Pivots per lane group when `kend` of them are dealt to `groups` groups in
+// runs, in steps of `step` (a lane's 16 bytes).
+__device__ __forceinline__ int run_length(int kend, int groups, int step) {
+    return (kend + groups * step - 1) / (groups * step) * step;
+}
+
 // U12 chunk product: G[i][j0 + jj] = (L11^-1 Ch)[i][jj] for i < K, jj < jn,
-// Li = L11^-1 in LDS (row stride kLinvLd), Ch the A12 chunk in LDS (row
-// stride kXCld, zero beyond K rows), four waves (FP32 or FP64 MFMA).
+// Lo = L11^-1 (global, [64][64], zero above the diagonal, unit beyond K), Ch
+// the A12 chunk in LDS (row stride kXCld, zero beyond K rows), four waves
+// (FP32 or FP64 MFMA).  A lane takes its row's operands as one run of pivots,
+// 16 bytes a load, all in flight at once, and no more of them than the strip's
+// triangle and the front's pivots need: staging the whole inverse in LDS first
+// cost 32 KiB of loads and of LDS per chunk in FP64 (two workgroups per CU
+// instead of four) whatever the pivot count.
 template <typename T>
-__device__ __forceinline__ void u12_product(const T* __restrict__ Li, const T* __restrict__ Ch,
+__device__ __forceinline__ void u12_product(const T* __restrict__ Lo, const T* __restrict__ Ch,
                                             T* __restrict__ G, int fs, int K, int j0, int jn) {
     const int lane = int(threadIdx.x) & 63, wave = int(threadIdx.x) >> 6;
+    constexpr int V = 16 / int(sizeof(T));
+    typedef T Run __attribute__((ext_vector_type(V)));
+    constexpr int NOP = sizeof(T) == 4 ? 32 : 16;
+    T a[NOP];
+    // rows at most `last`: operands k < min(K, last + 1)
+    auto load = [&](int row, int kend, int groups, int q) {
+        const int kw = run_length(kend, groups, V);
+        const Run* src = reinterpret_cast<const Run*>(Lo + row * kXMaxK + kw * q);
+#pragma unroll
+        for (int i = 0; i < NOP; i += V) {
+            if (i < kw) {                              // uniform
+                const Run v = src[i / V];
+#pragma unroll
+                for (int t = 0; t < V; ++t) a[i + t] = v[t];
+            }
+        }
+        return kw;
+    };
     if constexpr (sizeof(T) == 4) {
-        // 64 x 64 output = 2 x 2 tiles of 32 x 32, one per wave; L11^-1 is
-        // lower triangular, so the top row half needs k < 32 only
+        // 64 x 64 output = 2 x 2 tiles of 32 x 32, one per wave
         const int rh = wave & 1, ct = wave >> 1;
         if (32 * ct < jn && 32 * rh < K) {  // wave-uniform
             floatx16 acc;
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[v] = 0.f;
-            const int kend = rh == 0 ? 32 : 64;
-            for (int kk = 0; kk < kend; kk += 2) {
-                const int k = kk + (lane >> 5);
-                const float av = Li[(32 * rh + (lane & 31)) * kLinvLd + k];
-                const float bv = Ch[k * kXCld + 32 * ct + (lane & 31)];
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc, 0, 0, 0);
+            const int h = lane >> 5;
+            const int kw = load(32 * rh + (lane & 31), min(K, 32 * rh + 32), 2, h);
+#pragma unroll
+            for (int i = 0; i < NOP; ++i) {
+                if (i < kw) {                          // uniform
+                    const float bv = Ch[(kw * h + i) * kXCld + 32 * ct + (lane & 31)];
+                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], bv, acc, 0, 0, 0);
+                }
             }
             const int j = j0 + 32 * ct + (lane & 31);
 #pragma unroll
@@ -1092,22 +1122,22 @@ __device__ __forceinline__ void u12_product(const T* __restrict__ Li, const T* _
         }
     } else {
         // FP64 MFMA: 64 x 64 output = 4 x 4 tiles of 16 x 16, wave w the
-        // 16-row strip w; L11^-1 is lower (zero above the diagonal, unit
-        // beyond K, where the chunk rows are zero), so k < 16 w + 16
+        // 16-row strip w
         if (16 * wave < K) {                           // wave-uniform
             doublex4 acc[4];
 #pragma unroll
             for (int c = 0; c < 4; ++c) acc[c] = doublex4{0.0, 0.0, 0.0, 0.0};
-            const int r = 16 * wave + (lane & 15), q = lane >> 4;
-            const int kend = min(K, 16 * wave + 16);
-            for (int kk = 0; kk < kend; kk += 4) {
-                const int k = kk + q;
-                const double av = Li[r * kLinvLd + k];
+            const int q = lane >> 4;
+            const int kw = load(16 * wave + (lane & 15), min(K, 16 * wave + 16), 4, q);
 #pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    if (16 * c < jn) {                 // uniform
-                        const double bv = Ch[k * kXCld + 16 * c + (lane & 15)];
-                        acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[c], 0, 0, 0);
+            for (int i = 0; i < NOP; ++i) {
+                if (i < kw) {                          // uniform
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        if (16 * c < jn) {             // uniform
+                            const double bv = Ch[(kw * q + i) * kXCld + 16 * c + (lane & 15)];
+                            acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], bv, acc[c], 0, 0, 0);
+                        }
                     }
                 }
             }
@@ -1134,8 +1164,7 @@ __device__ __forceinline__ void u12_chunk(const LuDevice& d, const int* __restri
                                           const Arenas<T>& ar, const T* __restrict__ side, int fi,
                                           int ch, int b) {
     extern __shared__ unsigned char smem_raw[];
-    T* Li = reinterpret_cast<T*>(smem_raw);                        // [64][kLinvLd]
-    T* Ch = Li + 64 * kLinvLd;                                    // [64][kXCld]
+    T* Ch = reinterpret_cast<T*>(smem_raw);                       // [64][kXCld]
     const int p = fronts[fi];
     const int fs = d.fsz[p], K = d.nc[p];
     const int j0 = K + ch * kXChunk;
@@ -1144,9 +1173,6 @@ __device__ __forceinline__ void u12_chunk(const LuDevice& d, const int* __restri
     T* G = ar.a1 + (long long)b * d.arena1 + d.off[p];
     const int* rl = d.row_lb + d.lb_ptr[p];
     const T* Lo = side + ((long long)fi * Bp + b) * kSideElems + kUinvElems;
-    T lv[kUinvElems / kPivThreads];             // L11^-1, in flight during the assembly
-#pragma unroll
-    for (int u = 0; u < kUinvElems / kPivThreads; ++u) lv[u] = Lo[tid + u * kPivThreads];
     {
         const int jn = min(kXChunk, fs - j0);
         for (int e = tid; e < 64 * kXCld; e += kPivThreads) Ch[e] = T(0);
@@ -1158,13 +1184,8 @@ __device__ __forceinline__ void u12_chunk(const LuDevice& d, const int* __restri
         lds_barrier();
         assemble_chunks<kPivThreads, kAsmDepth>(d, ar, d.asm_base[p * kAsmKindCount + kAsmKChunk] + ch, b, Bp, Ch,
                                          [=](int r, int c) { return r * kXCld + c - j0; });
-#pragma unroll
-        for (int u = 0; u < kUinvElems / kPivThreads; ++u) {
-            const int e = tid + u * kPivThreads;
-            Li[(e >> 6) * kLinvLd + (e & 63)] = lv[u];
-        }
         lds_barrier();
-        u12_product<T>(Li, Ch, G, fs, K, j0, jn);
+        u12_product<T>(Lo, Ch, G, fs, K, j0, jn);
     }
 }
 
@@ -1535,8 +1556,7 @@ __global__ __launch_bounds__(kPivThreads) void k_chain_u12(LuDevice d, ChainDevi
                                                            int Bp, Arenas<float> ar,
                                                            const float* __restrict__ side, int nch) {
     extern __shared__ unsigned char smem_raw[];
-    float* Li = reinterpret_cast<float*>(smem_raw);               // [64][kLinvLd]
-    float* Chk = Li + 64 * kLinvLd;                               // [64][kXCld]
+    float* Chk = reinterpret_cast<float*>(smem_raw);              // [64][kXCld]
     int chn, b;
     decode_chain(nch, chn, b);
     const int p = ch.fronts[k];
@@ -1549,13 +1569,12 @@ __global__ __launch_bounds__(kPivThreads) void k_chain_u12(LuDevice d, ChainDevi
     const float* Tk = chain_base(d, ch, arena, ldT) + (long long)o * ldT + o;
     const float* Lo = side + (long long)b * kSideElems + kUinvElems;
     const int jn = min(kXChunk, fs - j0);
-    for (int e = tid; e < kUinvElems; e += kPivThreads) Li[(e >> 6) * kLinvLd + (e & 63)] = Lo[e];
     for (int e = tid; e < 64 * kXCld; e += kPivThreads) {
         const int r = e / kXCld, c = e - r * kXCld;
         Chk[e] = (r < K && c < jn) ? Tk[(long long)r * ldT + j0 + c] : 0.f;
     }
     lds_barrier();
-    u12_product<float>(Li, Chk, arena + d.off[p], fs, K, j0, jn);
+    u12_product<float>(Lo, Chk, arena + d.off[p], fs, K, j0, jn);
 }
 
 template <int MODE>
@@ -1767,14 +1786,17 @@ __device__ __forceinline__ void l21_block(const LuDevice& d, const int* __restri
             floatx16 acc;
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[v] = 0.f;
-            const int j = 32 * ct + (lane & 31);
-            const int kend = min(K, 32 * ct + 32);           // U11^-1 upper: k <= j
-            for (int kk = 0; kk < kend; kk += 2) {
-                const int k = kk + (lane >> 5);
-                const float av = Ab[(32 * rt + (lane & 31)) * kL21Ld + k];
-                const float bv = (k < K && j < K) ? float(Ui[k * kXMaxK + j]) : 0.f;
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc, 0, 0, 0);
-            }
+            const int j = 32 * ct + (lane & 31), h = lane >> 5;
+            const int kw = run_length(min(K, 32 * ct + 32), 2, 1);   // U11^-1 upper: k <= j
+            float u[32];
+#pragma unroll
+            for (int i = 0; i < 32; ++i)
+                if (i < kw) u[i] = Ui[(kw * h + i) * kXMaxK + j];     // uniform
+#pragma unroll
+            for (int i = 0; i < 32; ++i)
+                if (i < kw)
+                    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                        Ab[(32 * rt + (lane & 31)) * kL21Ld + kw * h + i], u[i], acc, 0, 0, 0);
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int r = 32 * rt + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);
@@ -1782,31 +1804,29 @@ __device__ __forceinline__ void l21_block(const LuDevice& d, const int* __restri
             }
         }
     } else {
-        // 64 x 64 = 4 x 4 tiles of 16 x 16; wave w: the 16-row strip w
+        // 64 x 64 = 4 x 4 tiles of 16 x 16; wave w: the 16-row strip w.  A
+        // tile's U11^-1 operands (k <= j; unit beyond K, where A21 is zero) all
+        // load before its products: one latency a tile, not one a step.
         if (16 * wave < nr) {                               // wave-uniform
-            doublex4 acc[4];
-#pragma unroll
-            for (int c = 0; c < 4; ++c) acc[c] = doublex4{0.0, 0.0, 0.0, 0.0};
             const int r = 16 * wave + (lane & 15), q = lane >> 4;
-            for (int kk = 0; kk < K; kk += 4) {
-                const int k = kk + q;
-                const double av = k < K ? double(Ab[r * kL21Ld + k]) : 0.0;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    if (16 * c < K) {                       // uniform
-                        const int j = 16 * c + (lane & 15);
-                        const double bv = (k < K && j < K) ? double(Ui[k * kXMaxK + j]) : 0.0;
-                        acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc[c], 0, 0, 0);
-                    }
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
+#pragma unroll 1
+            for (int c = 0; 16 * c < K; ++c) {              // uniform
                 const int j = 16 * c + (lane & 15);
+                const int kw = run_length(min(K, 16 * c + 16), 4, 1);
+                T u[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if (i < kw) u[i] = Ui[(kw * q + i) * kXMaxK + j];
+                doublex4 acc{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if (i < kw)
+                        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(double(Ab[r * kL21Ld + kw * q + i]),
+                                                                   double(u[i]), acc, 0, 0, 0);
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
                     const int rr = 16 * wave + q + 4 * v;
-                    if (rr < nr && j < K) G[(long long)(i0 + rr) * fs + j] = T(acc[c][v]);
+                    if (rr < nr && j < K) G[(long long)(i0 + rr) * fs + j] = T(acc[v]);
                 }
             }
         }
