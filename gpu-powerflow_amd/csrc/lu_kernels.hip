@@ -3,11 +3,12 @@
 // The fronts of one tree level are independent; the host launches one kernel
 // per (level, tier) group, children before parents.  Three tiers:
 //
-//   tier 0  fsz <= 16: batch-SIMT.  One wave = one front x 64 scenarios, one
-//           lane per scenario; the front lives in the scenario-interleaved
-//           arena (element e of scenario b at (off + e) * Bp + b), so every
-//           access of the wave is one contiguous segment and all control flow
-//           and index loads are wave-uniform.  No synchronisation at all.
+//   tier 0  fsz <= 16: batch-SIMT.  One workgroup = one front x 64 scenarios,
+//           one lane per scenario, the front's elements dealt to its waves;
+//           factored in LDS and stored to the scenario-interleaved arena
+//           (element e of scenario b at (off + e) * Bp + b), so every access
+//           of a wave is one contiguous segment and all control flow and
+//           index loads are wave-uniform.
 //   tier 1  fsz <= tier1_max, at most 32 pivots: one workgroup per (front,
 //           scenario); the front is assembled and factored in LDS and stored
 //           scenario-major.
@@ -207,7 +208,8 @@ __device__ __forceinline__ bool gate_closed(const int* gate) { return gate && *g
 // one row a wave at a time; last, the factored fronts go to the interleaved
 // arena.  Bound by the chain of LDS accesses of a wave's rows, and by the one
 // workgroup per CU that a 16-row FP64 front's 128 KiB leave: 16 waves for
-// fronts above kT0WideRows, four for smaller ones.
+// fronts above kT0WideRows, four for smaller ones (FP64 fronts of 12 to 16
+// rows: 469 us a launch by one wave in global memory, 130 so).
 template <typename T, int W>
 __global__ __launch_bounds__(64 * W) void k_factor_t0(LuDevice d, const int* __restrict__ fronts,
                                                       const double* __restrict__ A, int Bp,
@@ -1074,7 +1076,8 @@ __device__ __forceinline__ int run_length(int kend, int groups, int step) {
 // 16 bytes a load, all in flight at once, and no more of them than the strip's
 // triangle and the front's pivots need: staging the whole inverse in LDS first
 // cost 32 KiB of loads and of LDS per chunk in FP64 (two workgroups per CU
-// instead of four) whatever the pivot count.
+// instead of four) whatever the pivot count: 183 -> 135 us a launch in FP64,
+// 104 -> 78 in FP32 (2,000 buses x 1,024).
 template <typename T>
 __device__ __forceinline__ void u12_product(const T* __restrict__ Lo, const T* __restrict__ Ch,
                                             T* __restrict__ G, int fs, int K, int j0, int jn) {
@@ -1293,7 +1296,9 @@ __device__ __forceinline__ void cb_half_update(floatx16& acc, const U12Half<MODE
 
 // Three workgroups per CU: the 32 x 32 update tiles keep the kernel within
 // 168 VGPRs; the LDS (schur_lds) allows three up to 392 contribution columns
-// at <= 32 pivots.
+// at <= 32 pivots.  KM = 32 where no front of the group has more pivots: half
+// the operand registers (120 VGPRs) and half the products (3xBF16, 16 to 24
+// pivots: 440 -> 374 us a launch).
 template <typename T, int MODE, int KM>
 __global__ __launch_bounds__(kSchurThreads, 3) void k_schur(LuDevice d, const int* __restrict__ fronts,
                                                          const double* __restrict__ A, int Bp,
@@ -1715,20 +1720,28 @@ __global__ __launch_bounds__(kChainThreads, 2) void k_chain_strips(LuDevice d, C
 //     16x16x4, a 16-row strip per wave).
 //   k_schur_tile (one workgroup per (tile, scenario), 256 lanes): one
 //     64 x 64 tile of the contribution block C = A22 - L21 U12.  The tile of
-//     A22 is assembled in LDS (entries, then the tile's chunk map) while each
-//     wave's L21 operands (its 32 rows, read from the front) are in flight;
-//     each wave then loads its U12 operands (32 columns) and forms its
-//     32 x 32 quarter on MFMA (FP32 32x32x2, 3xBF16 32x32x16, or FP64
-//     16x16x4 as 2 x 2 tiles, a 16-column half at a time with that half's
-//     U12 operands) starting from the assembled values, and writes it once.
-//     Holding only the L21 operands through the assembly keeps FP64 within
-//     168 VGPRs (three workgroups per CU) and FP32 within 97.
+//     A22 is assembled in LDS (entries, then the tile's chunk map); each wave
+//     then loads its operands (32 rows of L21, 32 columns of U12) and forms
+//     its 32 x 32 quarter on MFMA (FP32 32x32x2, 3xBF16 32x32x16, or FP64
+//     16x16x4 as 2 x 2 tiles, eight pivots of a lane at a time) starting from
+//     the assembled values, and writes it once.  Loads return in order, so
+//     operands requested before the assembly would delay its loads; without
+//     them FP64 takes 113 VGPRs (four workgroups per CU).
+//     Bound by the assembly's chain of dependent loads (chunk, child element,
+//     LDS) in a workgroup's 20 to 40 us, four to a CU.  2,000 buses x 1,024,
+//     FP64: the levels with at most 32 pivots went from 2.18, 1.05, 0.85 and
+//     0.50 to 1.48, 0.69, 0.54 and 0.28 ms; those with 64 lost a tenth (1.17
+//     to 1.30, 0.81 to 0.92 ms), and the solve went from 97.0 to 84.6 ms with
+//     the other tier-2 kernels.  A form with all 64 pivots' operands in
+//     registers for the groups that need them, at three workgroups per CU,
+//     did not bring the tenth back.
 //
 // The operands' k index is split by lane group so every lane reads a run of
-// contiguous L21 elements: in an FP32 32x32x2 instruction i, lane half h
-// carries k = 32 h + i; in a 3xBF16 32x32x16 instruction j, k = 32 h + 8 j +
-// t (t < 8); in an FP64 16x16x4 instruction i, lane quarter q carries
-// k = 16 q + i.  FP64 16x16x4 layouts (checked on gfx950): A lane l = row
+// kw contiguous L21 elements, kw being the pivots dealt to a group (K over
+// the groups, in whole 16-byte runs): in an FP32 32x32x2 instruction i, lane
+// half h carries k = kw h + i; in a 3xBF16 32x32x16 instruction j, k = kw h +
+// 8 j + t (t < 8); in an FP64 16x16x4 instruction i, lane quarter q carries
+// k = kw q + i.  FP64 16x16x4 layouts (checked on gfx950): A lane l = row
 // l % 16, k = l / 16; B lane l = column l % 16, same k; accumulator register
 // v of lane l holds row l / 16 + 4 v, column l % 16.  The MFMA sums over every k of an instruction, so any
 // assignment shared by both operands gives the same product.

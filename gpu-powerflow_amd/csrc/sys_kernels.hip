@@ -15,7 +15,7 @@
 // What bounds it is the chain of dependent instructions (a wave alone on its
 // SIMD issues one about every 9 cycles): on 118 buses FP64 a Newton step takes
 // 69 us, 45 of them the 43 + 20 pivots of its levels one after another, 16 the
-// solve.  Solves: 118 buses x1 FP64 1.92 -> 0.43 ms (captured mixed 1.67 ->
+// solve.  Solves: 118 buses x1 FP64 1.92 -> 0.40 ms (captured mixed 1.67 ->
 // 0.33), x300 mixed 2.73 -> 0.48, x1,024 FP64 3.14 -> 1.41.
 #include "sys_kernels.hpp"
 #include "hip_common.hpp"
