@@ -286,8 +286,7 @@ def case118(torch, cupf, syn, po, args):
     """One scenario at a time on the 118-bus grid (GPU solve through the
     reference's single-scenario solve() with host arrays, and the device-
     resident batch entry at batch 1, eager and on the captured Newton step;
-    batch 1 runs the single-system LU kernels) against the oracle on one
-    core."""
+    whole Newton steps in one workgroup) against the oracle on one core."""
     g = syn.workload_grid("case118")
     n = g.n_bus
     N = 64
