@@ -16,15 +16,6 @@ namespace cupf {
 constexpr int kTier1MaxRows32 = CUPF_TIER1_ROWS32;
 constexpr int kTier1MaxRows64 = 90;
 
-// Panel cap of the plan where the caller asks for less (the options' default
-// is 8).  Narrow panels cut a separator into a chain of fronts that are
-// assembled and factored one after another, a level each: the 2,000-bus plan
-// has 68 levels and 5.9 M front elements at 8, 15 and 1.6 M at 64.  Solves at
-// 8 and 64: 501 buses mixed x257 6.7 and 4.3 ms, 1,000 buses mixed x300 14.1
-// and 7.7, 2,000 buses FP64 x256 79.8 and 29.4, 400 buses FP64 x1 6.4 and 4.5,
-// 118 buses mixed x4,000 3.57 and 3.08.  Wider caps are taken as they are.
-constexpr int kLeastCap = 64;
-
 // neighbouring scenarios that run each contribution-block tile together
 // (1, 4 and 16 measured alike on the 2,000-bus batch)
 constexpr int kTileScenGroup = 4;
@@ -49,7 +40,6 @@ void BatchedLU::analyze(int n, const int* rp, const int* ci, const std::vector<i
     if (opt.cap < 1) throw std::invalid_argument("BatchedLU::analyze(): panel cap must be >= 1");
     n_ = 0;
     opt_ = opt;
-    opt_.cap = std::max(opt.cap, kLeastCap);
     if (!aux_) {
         CUPF_HIP(hipStreamCreate(&aux_));
         CUPF_HIP(hipEventCreateWithFlags(&ev_fork_, hipEventDisableTiming));
@@ -263,8 +253,10 @@ void BatchedLU::analyze(int n, const int* rp, const int* ci, const std::vector<i
     nnz_ = nnz;
 }
 
-// Panel cap of the one-workgroup plan: its fronts are blocked by 16 pivots
-// whatever their width, so wide panels only save levels.
+// Panel cap of the one-workgroup plan, whatever the caller's (which shapes the
+// level sweeps): a workgroup eliminates a front pivot by pivot at any width, so
+// narrow panels only add levels and assemblies (118 buses: 9 levels and 10,032
+// additions at 8, 5 and 5,376 at 64).
 constexpr int kSysCap = 64;
 
 // Largest batch of the one-workgroup kernels.  They run a scenario per

@@ -484,6 +484,13 @@ int cupf_solver_debug_pattern(cupf_solver* solver, int32_t* row_ptr, int32_t* co
     return guarded([&] { solver_of(solver).debug_pattern(row_ptr, col_idx, perm); });
 }
 
+int cupf_solver_debug_plan(cupf_solver* solver, int32_t* out4) {
+    return guarded([&] {
+        if (!out4) throw std::invalid_argument("null argument");
+        solver_of(solver).debug_plan(out4);
+    });
+}
+
 int cupf_analyze_jacobian(int32_t n_bus, const int32_t* indptr, const int32_t* indices,
                           const int32_t* pv, int32_t n_pv, const int32_t* pq, int32_t n_pq,
                           int32_t* dim, int32_t* nnz, int32_t* row_ptr, int32_t* col_idx,

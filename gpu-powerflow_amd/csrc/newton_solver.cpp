@@ -1385,3 +1385,13 @@ void NewtonSolver::debug_pattern(int32_t* row_ptr, int32_t* col_idx, int32_t* pe
     std::copy(m.js.col_idx.begin(), m.js.col_idx.end(), col_idx);
     std::copy(m.lu.plan().perm.begin(), m.lu.plan().perm.end(), perm);
 }
+
+void NewtonSolver::debug_plan(int32_t* out4) const {
+    const Impl& m = *impl_;
+    if (!m.initialized) throw std::runtime_error("debug_plan: not initialized");
+    const SysPlan& p = m.lu.sys_plan();
+    out4[0] = m.lu.plan().num_fronts;
+    out4[1] = m.lu.plan().num_levels;
+    out4[2] = p.ok ? p.num_fronts : 0;
+    out4[3] = p.ok ? p.num_levels : 0;
+}

@@ -122,6 +122,9 @@ public:
                             double* x, uint8_t* singular);
     // Jacobian pattern and fill-reducing order of the last initialize().
     void debug_pattern(int32_t* row_ptr, int32_t* col_idx, int32_t* perm) const;
+    // Fronts and levels of the level sweeps' plan, then of the one-workgroup
+    // plan (0, 0: the system does not qualify).
+    void debug_plan(int32_t* out4) const;
 
 private:
     struct Impl;

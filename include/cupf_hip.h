@@ -234,6 +234,9 @@ int cupf_solver_debug_factor_solve(cupf_solver* solver, const double* A, const d
                                    uint8_t* singular);
 int cupf_solver_debug_pattern(cupf_solver* solver, int32_t* row_ptr, int32_t* col_idx,
                               int32_t* perm);
+/* fronts and levels of the level sweeps' plan, then of the one-workgroup plan
+ * (0, 0: the system does not qualify for it) */
+int cupf_solver_debug_plan(cupf_solver* solver, int32_t out4[4]);
 
 /* ---- Host analysis (no GPU needed) ------------------------------------ */
 /* Jacobian pattern + scatter maps; the reference's make_jacobian_indexing /

@@ -163,3 +163,10 @@ def debug_factor_solve(handle, A, rhs, transpose=False):
                                                ctypes.c_int32(1 if transpose else 0), _p(x),
                                                _p(sing)))
     return x, sing
+
+
+def debug_plan(handle):
+    """Fronts and levels of the level sweeps' and the one-workgroup plan."""
+    out = np.zeros(4, np.int32)
+    check(lib().cupf_solver_debug_plan(_h(handle), _p(out)))
+    return dict(zip(("fronts", "levels", "sys_fronts", "sys_levels"), out.tolist()))

@@ -110,3 +110,24 @@ def test_small_pivots_are_replaced_and_flagged(gpu, cupf, syn, oracle):
     want[7, 3], want[9, 3] = 1e8, -1e8
     np.testing.assert_allclose(x, want, rtol=1e-15)
     assert sing[7] and sing[9] and sing.sum() == 2
+
+
+def test_panel_cap_shapes_the_level_sweeps_only(gpu, cupf, syn):
+    """The level sweeps' plan is the caller's cap's; the one-workgroup plan is
+    the same at every cap, and so are its results to the bit."""
+    g = syn.workload_grid("case118")
+    a = capi.analyze_jacobian(g.n_bus, g.indptr, g.indices, g.pv, g.pq)
+    perm = capi.order_jacobian(g.n_bus, g.indptr, g.indices, g.pv, g.pq, a["dim"])
+    fronts = {cap: capi.plan_figures(a["row_ptr"], a["col_idx"], perm, cap)["fronts"] for cap in (8, 64, 128)}
+    assert fronts[8] > fronts[64]
+    S = g.sbus_scaled(syn.load_factors(65, g.n_bus, 0.7, 1.3, 2))
+    V0 = g.flat_start(65)
+    sys_plan, V = set(), []
+    for cap in (8, 64, 128):
+        s = _solver(cupf, g, "FP64", cap)
+        plan = capi.debug_plan(s.handle)
+        assert plan["fronts"] == fronts[cap]
+        sys_plan.add((plan["sys_fronts"], plan["sys_levels"]))
+        V.append(s.solve_batch(g.indptr, g.indices, g.data, g.n_bus, g.n_bus, S, V0, g.pv, g.pq).V_numpy)
+    assert sys_plan == {(fronts[64], 5)}
+    assert (V[0] == V[1]).all() and (V[0] == V[2]).all()
