@@ -253,12 +253,6 @@ void BatchedLU::analyze(int n, const int* rp, const int* ci, const std::vector<i
     nnz_ = nnz;
 }
 
-// Panel cap of the one-workgroup plan, whatever the caller's (which shapes the
-// level sweeps): a workgroup eliminates a front pivot by pivot at any width, so
-// narrow panels only add levels and assemblies (118 buses: 9 levels and 10,032
-// additions at 8, 5 and 5,376 at 64).
-constexpr int kSysCap = 64;
-
 // Largest batch of the one-workgroup kernels.  They run a scenario per
 // workgroup, one to seven workgroups to a CU by their LDS, so their time grows
 // by the rounds of workgroups; the level sweeps cost some 0.5 ms a Newton step
@@ -273,12 +267,10 @@ void BatchedLU::find_sys(int n_bus, const int* rp, const int* ci, const std::vec
                          hipStream_t s) {
     sys_ = SysPlan{};
     sys_dev_ = kern::SysDevice{};
-    // fronts only grow with the cap, so a narrower plan's tell already
-    if (opt_.cap <= kSysCap && plan_.max_fsz > kSysMaxRows) return;
-    const LuPlan P = opt_.cap == kSysCap ? plan_ : lower_plan(analyze_symbolic(sym_.n, rp, ci, perm, kSysCap), sym_.n, rp, ci);
-    sys_ = make_sys_plan(P, kern::kSysLdsMax / front_bytes());
+    sys_ = find_sys_plan(plan_, opt_.cap, rp, ci, perm, kern::kSysLdsMax / front_bytes());
+    if (!sys_.ok) return;
     sys_lds_ = kern::sys_lds_bytes(sys_, int(front_bytes()), 0);
-    if (!sys_.ok || kern::sys_lds_bytes(sys_, int(front_bytes()), n_bus) > kern::kSysLdsMax) {
+    if (kern::sys_lds_bytes(sys_, int(front_bytes()), n_bus) > kern::kSysLdsMax) {
         sys_.ok = false;
         return;
     }
@@ -299,7 +291,6 @@ void BatchedLU::find_sys(int n_bus, const int* rp, const int* ci, const std::vec
     d.blob = d_sys_blob.as<int4>();
     d.slot_pos = d_sys_slot.as<int>();
 }
-
 
 int BatchedLU::scenarios(int Bp) const {
     if (B_ < 1 || B_ > Bp || B_ <= Bp - kern::kLanes)

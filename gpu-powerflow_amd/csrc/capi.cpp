@@ -560,6 +560,22 @@ int cupf_plan_figures(int32_t n, const int32_t* row_ptr, const int32_t* col_idx,
     });
 }
 
+int cupf_plan_sys(int32_t n, const int32_t* row_ptr, const int32_t* col_idx, const int32_t* perm,
+                  int32_t cap, int32_t elem, int32_t* out3) {
+    return guarded([&] {
+        if (!row_ptr || !col_idx || !perm || !out3) throw std::invalid_argument("null argument");
+        if (elem != 4 && elem != 8) throw std::invalid_argument("cupf_plan_sys: elements of 4 or 8 bytes");
+        const std::vector<int> pv(perm, perm + n);
+        const cupf::Symbolic s = cupf::analyze_symbolic(n, row_ptr, col_idx, pv, cap);
+        const cupf::LuPlan p = cupf::lower_plan(s, n, row_ptr, col_idx);
+        const cupf::SysPlan q =
+            cupf::find_sys_plan(p, cap, row_ptr, col_idx, pv, cupf::kern::kSysLdsMax / size_t(elem));
+        out3[0] = q.ok ? q.num_fronts : 0;
+        out3[1] = q.ok ? q.num_levels : 0;
+        out3[2] = q.ok ? q.fac + q.scratch : 0;
+    });
+}
+
 int cupf_plan_chains(int32_t n, const int32_t* row_ptr, const int32_t* col_idx,
                      const int32_t* perm, int32_t cap, int32_t* sizes, int32_t max_sizes,
                      int32_t* out2) {

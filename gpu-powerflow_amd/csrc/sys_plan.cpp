@@ -50,11 +50,21 @@ SysPlan make_sys_plan(const LuPlan& P, size_t most_elems) {
     std::vector<int> order(static_cast<size_t>(F));
     for (int p = 0; p < F; ++p) order[size_t(p)] = p;
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return P.level[a] < P.level[b]; });
+    // sizes first: a system that is too large costs one pass over its fronts,
+    // and the allocation below (fronts squared) ends where the blocks no longer fit
+    for (int p = 0; p < F; ++p) {
+        const int fs = P.fsz[p], K = P.nc[p], uc = fs - K;
+        fac += (long long)K * (fs | 1) + (long long)uc * (K | 1);
+        work += fs;
+    }
+    if (size_t(fac + work) > most_elems) return S;
     for (int p : order) {
         const int fs = P.fsz[p], K = P.nc[p], uc = fs - K;
         const int to = parent[size_t(p)] >= 0 ? P.level[parent[size_t(p)]] : P.level[p];
         fr[size_t(p)].co = arena.take(uc * uc, P.level[p], to);
+        if (size_t(fac + arena.top) > most_elems) return S;
     }
+    fac = work = 0;
     for (int p = 0; p < F; ++p) {
         const int fs = P.fsz[p], K = P.nc[p], uc = fs - K;
         SysFront& f = fr[size_t(p)];
@@ -194,6 +204,16 @@ SysPlan make_sys_plan(const LuPlan& P, size_t most_elems) {
     }
     S.ok = true;
     return S;
+}
+
+SysPlan find_sys_plan(const LuPlan& P, int cap, const int* rp, const int* ci, const std::vector<int>& perm,
+                      size_t most_elems) {
+    // Entries of L and U off the diagonal: the least elements of the factors at
+    // any cap, known without another analysis.  Fronts only grow with the cap,
+    // so those of a narrower plan tell too.
+    if (size_t(2 * (P.lnz - P.n)) > most_elems || (cap <= kSysCap && P.max_fsz > kSysMaxRows)) return SysPlan{};
+    if (cap == kSysCap) return make_sys_plan(P, most_elems);
+    return make_sys_plan(lower_plan(analyze_symbolic(P.n, rp, ci, perm, kSysCap), P.n, rp, ci), most_elems);
 }
 
 }  // namespace cupf

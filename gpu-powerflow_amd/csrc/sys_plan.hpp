@@ -62,7 +62,18 @@ constexpr int kSysSmallRows = 16;
 // largest front (the shared fronts' register tiles)
 constexpr int kSysMaxRows = 112;
 
+// Panel cap of the one-workgroup plan, whatever the caller's (which shapes the
+// level sweeps): a workgroup eliminates a front pivot by pivot at any width, so
+// narrow panels only add levels and assemblies (118 buses: 9 levels at 8, 5 at
+// 64).
+constexpr int kSysCap = 64;
+
 // most_elems: elements (factors and scratch) that may fit the LDS at all.
 SysPlan make_sys_plan(const LuPlan& P, size_t most_elems);
+
+// The one-workgroup plan (ok false: the system does not qualify) of the pattern
+// rp/ci in the order perm, whose plan at the caller's cap is P.
+SysPlan find_sys_plan(const LuPlan& P, int cap, const int* rp, const int* ci, const std::vector<int>& perm,
+                      size_t most_elems);
 
 }  // namespace cupf

@@ -271,6 +271,13 @@ int cupf_symbolic(int32_t n, const int32_t* row_ptr, const int32_t* col_idx,
 int cupf_plan_figures(int32_t n, const int32_t* row_ptr, const int32_t* col_idx,
                       const int32_t* perm, int32_t cap, double* out5);
 
+/* The one-workgroup plan of (pattern, perm) for a solver at panel cap `cap`
+ * with fronts of `elem` bytes an element (host analysis only; no reference
+ * counterpart): out3 = {fronts, levels, elements in LDS}, zeros when the system
+ * does not qualify. */
+int cupf_plan_sys(int32_t n, const int32_t* row_ptr, const int32_t* col_idx, const int32_t* perm,
+                  int32_t cap, int32_t elem, int32_t* out3);
+
 /* Chains of nested fronts of the lowered plan (FP32 fronts) for (pattern,
  * perm, cap): fronts whose contribution rows are exactly their parent's rows,
  * factored in place by the chain kernels (host analysis only; no reference

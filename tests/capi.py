@@ -108,6 +108,15 @@ def plan_figures(row_ptr, col_idx, perm, cap):
             "lnz": int(out[4])}
 
 
+def plan_sys(row_ptr, col_idx, perm, cap, elem):
+    """The one-workgroup plan: fronts, levels and elements in LDS (0: none)."""
+    n = len(row_ptr) - 1
+    out = np.zeros(3, np.int32)
+    check(lib().cupf_plan_sys(ctypes.c_int32(n), _p(_i32(row_ptr)), _p(_i32(col_idx)), _p(_i32(perm)),
+                              ctypes.c_int32(cap), ctypes.c_int32(elem), _p(out)))
+    return dict(zip(("fronts", "levels", "elems"), out.tolist()))
+
+
 def plan_chains(row_ptr, col_idx, perm, cap, max_sizes=256):
     """Chains of nested fronts of the FP32 plan: counts and the front sizes."""
     n = len(row_ptr) - 1

@@ -11,6 +11,8 @@ extend-add map) must then be identical.
 
 from __future__ import annotations
 
+import time
+
 import numpy as np
 import pytest
 
@@ -191,3 +193,34 @@ def test_nested_chain_of_the_2000_bus_plan(syn):
     fig = capi.plan_figures(a["row_ptr"], a["col_idx"], perm, 64)
     assert ch["sizes"][0] == fig["max_fsz"]          # the top separator's first panel
     assert capi.plan_chains(a["row_ptr"], a["col_idx"], perm, 1 << 20)["chains"] == 0
+
+
+def test_one_workgroup_plan_is_the_same_at_every_cap(syn):
+    g = syn.workload_grid("case118")
+    a = capi.analyze_jacobian(g.n_bus, g.indptr, g.indices, g.pv, g.pq)
+    perm = capi.order_jacobian(g.n_bus, g.indptr, g.indices, g.pv, g.pq, a["dim"])
+    plans = [capi.plan_sys(a["row_ptr"], a["col_idx"], perm, cap, 8) for cap in (1, 8, 64, 200)]
+    assert plans[0]["fronts"] == capi.plan_figures(a["row_ptr"], a["col_idx"], perm, 64)["fronts"]
+    assert all(p == plans[0] for p in plans)
+
+
+@pytest.mark.parametrize("cap", [8, 64, 128])
+def test_one_workgroup_plan_of_a_large_tree_is_refused_early(cap):
+    """A 20,000-bus radial network has small fronts only and far too many of
+    them: refusing it takes less than the analysis (twice its time and 100 ms
+    allow for a busy machine; laying the plan out first took nine times it)."""
+    n = 20000
+    rng = np.random.default_rng(1)
+    up = np.maximum(0, np.arange(1, n) - 1 - rng.integers(0, 8, n - 1))
+    ij = np.r_[np.c_[np.arange(n), np.arange(n)], np.c_[np.arange(1, n), up], np.c_[up, np.arange(1, n)]]
+    ij = np.unique(ij, axis=0)
+    indptr = np.r_[0, np.cumsum(np.bincount(ij[:, 0], minlength=n))]
+    pv, pq = np.arange(7, n, 7), np.setdiff1d(np.arange(1, n), np.arange(7, n, 7))
+    a = capi.analyze_jacobian(n, indptr, ij[:, 1], pv, pq)
+    perm = capi.order_jacobian(n, indptr, ij[:, 1], pv, pq, a["dim"])
+    t0 = time.perf_counter()
+    capi.plan_figures(a["row_ptr"], a["col_idx"], perm, cap)
+    t1 = time.perf_counter()
+    assert capi.plan_sys(a["row_ptr"], a["col_idx"], perm, cap, 4)["fronts"] == 0
+    t2 = time.perf_counter()
+    assert t2 - t1 <= 2 * (t1 - t0) + 0.1
