@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstddef>
 #include <stdexcept>
 #include <string>
@@ -17,6 +18,28 @@ inline void hip_check(hipError_t e, const char* what) {
 }
 
 #define CUPF_HIP(call) ::cupf::hip_check((call), #call)
+
+// Work done once per process and device, such as raising a kernel's LDS limit:
+// a bit per device (on devices past the word's, every time).
+class OncePerDevice {
+public:
+    template <class F>
+    void operator()(F work) {
+        int dev = 0;
+        CUPF_HIP(hipGetDevice(&dev));
+        const unsigned long long bit = dev < 64 ? 1ull << dev : 0;
+        if (done_.load(std::memory_order_acquire) & bit) return;
+        work();
+        done_.fetch_or(bit, std::memory_order_release);
+    }
+
+private:
+    std::atomic<unsigned long long> done_{0};
+};
+
+inline void raise_lds(const void* kernel, size_t bytes) {
+    CUPF_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
+}
 
 // Owning device allocation.  Moves, never copies.
 class DeviceBuffer {

@@ -2610,14 +2610,11 @@ void cross_group(const LuDevice& d, const int* fronts, int count, int max_fsz, c
                  int Bp, Arenas<T> ar, T* uinv, double pivot_eps, int static_piv, int* sing,
                  bool with_l21, hipStream_t s) {
     if (count <= 0) return;
-    static bool attr_set = false;
-    if (!attr_set) {
-        CUPF_HIP(hipFuncSetAttribute((const void*)k_pivot<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     int(pivot_lds<T>())));
-        CUPF_HIP(hipFuncSetAttribute((const void*)k_u12<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     int(u12_lds<T>())));
-        attr_set = true;
-    }
+    static OncePerDevice first_use;
+    first_use([&] {
+        raise_lds((const void*)k_pivot<T>, pivot_lds<T>());
+        raise_lds((const void*)k_u12<T>, u12_lds<T>());
+    });
     hipLaunchKernelGGL(k_pivot<T>, dim3(unsigned(count) * unsigned(d.nb)), dim3(pivot_threads<T>()),
                        pivot_lds<T>(), s, d,
                        fronts, A, Bp, ar, uinv, pivot_eps, static_piv, sing);
@@ -2642,13 +2639,10 @@ void cross_group(const LuDevice& d, const int* fronts, int count, int max_fsz, c
 template <typename T, int MODE, int KM>
 void launch_schur(const LuDevice& d, const int* fronts, const double* A, int Bp, Arenas<T> ar, const T* uinv,
                   int nrb, int sld, unsigned blocks, size_t shmem, hipStream_t s) {
-    static bool attr_set = false;
-    if (!attr_set) {
-        CUPF_HIP(hipFuncSetAttribute((const void*)k_schur<T, MODE, KM>,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     int(schur_lds<T>(kSLd, kDenseMaxFsz))));
-        attr_set = true;
-    }
+    static OncePerDevice first_use;
+    first_use([&] {
+        raise_lds((const void*)k_schur<T, MODE, KM>, schur_lds<T>(kSLd, kDenseMaxFsz));
+    });
     hipLaunchKernelGGL((k_schur<T, MODE, KM>), dim3(blocks), dim3(kSchurThreads), shmem, s, d, fronts, A, Bp,
                        ar, uinv, nrb, sld);
     CUPF_HIP(hipGetLastError());
@@ -2716,16 +2710,12 @@ void chain_factor(const LuDevice& d, const ChainDevice& c, const std::vector<int
     const size_t piv_lds = size_t(64 * kPivLd) * sizeof(float);
     const size_t u12_bytes = u12_lds<float>();
     const size_t strip_lds = size_t(64 * kLinvLd + kChainStrips * kChainStrip * kChainLd) * sizeof(float);
-    static bool attr_set = false;
-    if (!attr_set) {
-        CUPF_HIP(hipFuncSetAttribute((const void*)k_chain_u12, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     int(u12_bytes)));
-        CUPF_HIP(hipFuncSetAttribute((const void*)k_chain_strips<kMfmaF32>,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(strip_lds)));
-        CUPF_HIP(hipFuncSetAttribute((const void*)k_chain_strips<kMfmaBf16x3>,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(strip_lds)));
-        attr_set = true;
-    }
+    static OncePerDevice first_use;
+    first_use([&] {
+        raise_lds((const void*)k_chain_u12, u12_bytes);
+        raise_lds((const void*)k_chain_strips<kMfmaF32>, strip_lds);
+        raise_lds((const void*)k_chain_strips<kMfmaBf16x3>, strip_lds);
+    });
     int o = 0;
     for (int k = 1; k <= c.steps; ++k) {
         const int fs = fsz[size_t(k)], K = nc[size_t(k)], uc = fs - K;
@@ -2766,12 +2756,10 @@ void launch_t0(const LuDevice& d, const int* fronts, int count, int max_fsz, con
                Arenas<T> ar, double pivot_eps, int static_piv, int* sing, hipStream_t s) {
     constexpr size_t most = size_t(kTier0Max) * kTier0Max * kLanes * sizeof(T);
     static_assert(most <= 160 * 1024, "a tier-0 front of 64 scenarios in LDS");
-    static bool attr_set = false;
-    if (!attr_set) {
-        CUPF_HIP(hipFuncSetAttribute((const void*)k_factor_t0<T, W>,
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(most)));
-        attr_set = true;
-    }
+    static OncePerDevice first_use;
+    first_use([&] {
+        raise_lds((const void*)k_factor_t0<T, W>, most);
+    });
     const size_t shmem = size_t(max_fsz) * max_fsz * kLanes * sizeof(T);
     hipLaunchKernelGGL((k_factor_t0<T, W>), dim3(count, Bp / kLanes), dim3(64 * W), shmem, s, d, fronts, A, Bp,
                        ar, pivot_eps, static_piv, sing);
@@ -2785,14 +2773,11 @@ void lu_factor_group(const LuDevice& d, int tier, const int* fronts, int count, 
     if (tier == 2) assemble_rows<T>(d, fronts, count, max_fsz, A, Bp, ar, s);
     if constexpr (sizeof(T) == 4) {
     if (tier == 2 && dense_mode != 0 && max_fsz <= kDenseMaxFsz) {
-        static bool attr_set = false;
-        if (!attr_set) {
-            CUPF_HIP(hipFuncSetAttribute((const void*)k_factor_t2_mfma<kMfmaF32>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, int(kDenseLds)));
-            CUPF_HIP(hipFuncSetAttribute((const void*)k_factor_t2_mfma<kMfmaBf16x3>,
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, int(kDenseLds)));
-            attr_set = true;
-        }
+        static OncePerDevice first_use;
+        first_use([&] {
+            raise_lds((const void*)k_factor_t2_mfma<kMfmaF32>, kDenseLds);
+            raise_lds((const void*)k_factor_t2_mfma<kMfmaBf16x3>, kDenseLds);
+        });
         Arenas<float> af{reinterpret_cast<float*>(ar.a0), reinterpret_cast<float*>(ar.a1)};
         const dim3 grid(unsigned(count) * unsigned(d.nb));
         if (dense_mode == kMfmaBf16x3)

@@ -21,7 +21,6 @@
 #include "hip_common.hpp"
 
 #include <algorithm>
-#include <atomic>
 #include <type_traits>
 
 namespace cupf::kern {
@@ -904,12 +903,6 @@ __global__ __launch_bounds__(NT, 2) void k_sys_newton(SysDevice d, NrDevice nr, 
 constexpr int kSysWide = 512, kSysNarrow = 256;
 constexpr int kSysCus = 256;
 
-template <typename K>
-void raise_lds(K kernel) {
-    CUPF_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, int(kSysLdsMax)));
-}
-
 }  // namespace
 
 size_t sys_lds_bytes(const SysPlan& p, int elem, int n_bus) {
@@ -922,29 +915,26 @@ size_t sys_lds_bytes(const SysPlan& p, int elem, int n_bus) {
 
 template <int NT>
 void raise_all() {
-    raise_lds(k_sys_factor<double, NT>);
-    raise_lds(k_sys_factor<float, NT>);
-    raise_lds(k_sys_solve<double, false, double, NT>);
-    raise_lds(k_sys_solve<double, true, double, NT>);
-    raise_lds(k_sys_solve<double, false, float, NT>);
-    raise_lds(k_sys_solve<double, true, float, NT>);
-    raise_lds(k_sys_solve<float, false, double, NT>);
-    raise_lds(k_sys_solve<float, true, double, NT>);
-    raise_lds(k_sys_solve<float, false, float, NT>);
-    raise_lds(k_sys_solve<float, true, float, NT>);
-    raise_lds(k_sys_newton<double, NT>);
-    raise_lds(k_sys_newton<float, NT>);
+    raise_lds((const void*)k_sys_factor<double, NT>, kSysLdsMax);
+    raise_lds((const void*)k_sys_factor<float, NT>, kSysLdsMax);
+    raise_lds((const void*)k_sys_solve<double, false, double, NT>, kSysLdsMax);
+    raise_lds((const void*)k_sys_solve<double, true, double, NT>, kSysLdsMax);
+    raise_lds((const void*)k_sys_solve<double, false, float, NT>, kSysLdsMax);
+    raise_lds((const void*)k_sys_solve<double, true, float, NT>, kSysLdsMax);
+    raise_lds((const void*)k_sys_solve<float, false, double, NT>, kSysLdsMax);
+    raise_lds((const void*)k_sys_solve<float, true, double, NT>, kSysLdsMax);
+    raise_lds((const void*)k_sys_solve<float, false, float, NT>, kSysLdsMax);
+    raise_lds((const void*)k_sys_solve<float, true, float, NT>, kSysLdsMax);
+    raise_lds((const void*)k_sys_newton<double, NT>, kSysLdsMax);
+    raise_lds((const void*)k_sys_newton<float, NT>, kSysLdsMax);
 }
 
 void sys_prepare() {
-    static std::atomic<unsigned long long> done{0};             // a bit per device
-    int dev = 0;
-    CUPF_HIP(hipGetDevice(&dev));
-    const unsigned long long bit = 1ull << (dev & 63);
-    if (done.load(std::memory_order_acquire) & bit) return;
-    raise_all<kSysWide>();
-    raise_all<kSysNarrow>();
-    done.fetch_or(bit, std::memory_order_release);
+    static OncePerDevice first_use;
+    first_use([] {
+        raise_all<kSysWide>();
+        raise_all<kSysNarrow>();
+    });
 }
 
 // go(threads) with the workgroup size for B scenarios as a compile-time value

@@ -145,3 +145,39 @@ def test_integration_ctypes_snippets_match_the_header():
         assert _top_level_args(args) == arity[name], (name, args, arity[name])
         calls += 1
     assert calls >= 5
+
+
+def test_kernel_limits_are_raised_on_each_device(tmp_path):
+    """A kernel's LDS limit belongs to a device: OncePerDevice runs its work
+    once on each of three devices (the current device is the test's own
+    hipGetDevice), again after a failure, and no launcher keeps a flag of its
+    own for the whole process."""
+    csrc = capi.ROOT / "gpu-powerflow_amd" / "csrc"
+    src = tmp_path / "once.cpp"
+    src.write_text("""
+#include "hip_common.hpp"
+#include <cstdio>
+static int current = 0;
+extern "C" hipError_t hipGetDevice(int* d) { *d = current; return hipSuccess; }
+extern "C" const char* hipGetErrorString(hipError_t) { return ""; }
+int main() {
+    cupf::OncePerDevice once;
+    int runs[80] = {};
+    for (int pass = 0; pass < 2; ++pass)
+        for (int d : {0, 1, 63, 70})
+            for (int k = 0; k < 2; ++k) {
+                current = d;
+                try {
+                    once([&] { if (++runs[d] == 1 && d == 1) throw 1; });
+                } catch (int) {}
+            }
+    std::printf("%d %d %d %d\\n", runs[0], runs[1], runs[63], runs[70]);
+}
+""")
+    exe = tmp_path / "once"
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", f"-I{csrc}",
+                    str(src), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout
+    assert out.split() == ["1", "2", "1", "4"]
+    for f in csrc.glob("*.hip"):
+        assert "static bool" not in f.read_text(), f.name
