@@ -28,20 +28,38 @@ namespace {
 
 constexpr unsigned long long kNanBits = 0x7FF8000000000000ULL;
 
+// Pivots from least() up to most() have a reciprocal that is a normal number.
+__device__ __forceinline__ double least(double) { return 0x1p-1022; }
+__device__ __forceinline__ double most(double) { return 0x1p1022; }
+__device__ __forceinline__ float least(float) { return 0x1p-126f; }
+__device__ __forceinline__ float most(float) { return 0x1p126f; }
+
 // The pivot rule of the batched kernels without branches: |pivot| <= low
 // becomes +-rep and raises the flag (static pivots: both are eps; else a zero
-// pivot becomes 1).
+// pivot becomes 1).  Plain pivots are not replaced and have a reciprocal.
 template <typename T>
 struct PivotRule {
-    T low, rep;
+    T low, rep, floor;
     bool sign;
     __device__ __forceinline__ PivotRule(double eps, int static_piv)
-        : low(static_piv ? T(eps) : T(0)), rep(static_piv ? T(eps) : T(1)), sign(static_piv != 0) {}
+        : low(static_piv ? T(eps) : T(0)), rep(static_piv ? T(eps) : T(1)),
+          floor(low > least(T()) ? low : least(T())), sign(static_piv != 0) {}
     __device__ __forceinline__ bool small(T piv) const { return (piv < T(0) ? -piv : piv) <= low; }
     __device__ __forceinline__ T replaced(T piv) const { return sign && piv < T(0) ? -rep : rep; }
+    __device__ __forceinline__ bool plain(T piv) const {
+        const T m = piv < T(0) ? -piv : piv;
+        return m > floor && m < most(T());
+    }
+    // piv, or NaN (which the reciprocal hands on to the solves' quotients)
+    // where it has no reciprocal
+    __device__ __forceinline__ T divisor(T piv) const {
+        const T m = piv < T(0) ? -piv : piv;
+        return m >= least(T()) && m < most(T()) ? piv : T(__builtin_nanf(""));
+    }
 };
 
-// 1 / d by Newton's iteration from the hardware estimate, within an ulp.
+// 1 / d by Newton's iteration from the hardware estimate, within an ulp; NaN
+// for NaN.
 __device__ __forceinline__ double reciprocal(double d) {
     double r = __builtin_amdgcn_rcp(d);
     r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
@@ -52,15 +70,22 @@ __device__ __forceinline__ float reciprocal(float d) {
     return __builtin_fmaf(__builtin_fmaf(-d, r, 1.f), r, r);
 }
 
-// a / d from r = 1 / d: the product and one residual correction, within an
-// ulp of the division at a quarter of its latency.
-__device__ __forceinline__ double over(double a, double d, double r) {
+// a / d from r = 1 / d: the product and one residual correction, which round
+// as the division does (no difference in 10^8 pairs of either type) at a
+// quarter of its latency.  NaN where r is NaN, a is infinite or the quotient
+// overflows: the factorisations look at their pivots, the solves at their
+// results, and divide then.
+__device__ __forceinline__ double quotient(double a, double d, double r) {
     const double q = a * r;
     return __builtin_fma(__builtin_fma(-d, q, a), r, q);
 }
-__device__ __forceinline__ float over(float a, float d, float r) {
+__device__ __forceinline__ float quotient(float a, float d, float r) {
     const float q = a * r;
     return __builtin_fmaf(__builtin_fmaf(-d, q, a), r, q);
+}
+template <bool EXACT, typename T>
+__device__ __forceinline__ T over(T a, T d, T r) {
+    return EXACT ? a / d : quotient(a, d, r);
 }
 
 __device__ __forceinline__ double nfma(double a, double b, double c) { return __builtin_fma(-a, b, c); }
@@ -226,7 +251,7 @@ __device__ __forceinline__ void eliminate_step(T (&x)[16], int r, int K, const P
     }
     const T ri = reciprocal(piv);
     rinv = r == k ? ri : rinv;
-    const T l = over(below ? x[k] : T(0), piv, ri);
+    const T l = quotient(below ? x[k] : T(0), piv, ri);
     x[k] = below ? l : x[k];
     const T nl = -l;
 #pragma unroll
@@ -251,6 +276,31 @@ __device__ __forceinline__ void eliminate16(T (&x)[16], int r, int K, int kmax,
 __device__ __forceinline__ int over_groups(int v) {
     return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
                max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+
+// The same by division on the assembled fronts in LDS, for fronts with a pivot
+// that has no reciprocal.
+template <typename T>
+__device__ __forceinline__ void eliminate_dividing(const Sys<T>& S, const Front& f, int r, int fs, int K,
+                                                   int kmax, const PivotRule<T>& rule, int& flag) {
+    for (int k = 0; k < kmax; ++k) {
+        const bool on = k < K, below = on && r > k && r < fs;
+        T piv = on ? S.a[f.at(k, k)] : T(1);
+        const bool low = on && rule.small(piv);
+        flag |= low;
+        piv = low ? rule.replaced(piv) : piv;
+        wave_sync();
+        if (on && r == k) {
+            S.a[f.at(k, k)] = piv;
+            S.dinv[f.first + k] = reciprocal(rule.divisor(piv));
+        }
+        if (below) {
+            const T l = S.a[f.at(r, k)] / piv;
+            S.a[f.at(r, k)] = l;
+            for (int j = k + 1; j < fs; ++j) S.a[f.at(r, j)] = nfma(l, S.a[f.at(k, j)], S.a[f.at(r, j)]);
+        }
+        wave_sync();
+    }
 }
 
 // Four fronts of at most 16 rows, one per 16 lanes: contribution blocks added
@@ -280,7 +330,13 @@ __device__ __forceinline__ void factor_quad(const Sys<T>& S, const unsigned shor
         x[j] = r < fs && j < fs ? v : T(0);
     }
     T rinv = T(1);
-    eliminate16<0>(x, r, K, kmax, rule, flag, rinv);
+    int replaced = 0;
+    eliminate16<0>(x, r, K, kmax, rule, replaced, rinv);
+    if (__builtin_expect(__any(!__builtin_isnormal(rinv)), 0)) {
+        eliminate_dividing(S, f, r, fs, K, kmax, rule, flag);
+        return;
+    }
+    flag |= replaced;
 #pragma unroll
     for (int j = 0; j < 16; ++j)
         if (r < fs && j < fs) S.a[(j < f.K ? lo : hi) + j] = x[j];
@@ -346,20 +402,30 @@ __device__ __forceinline__ void factor_front(const Sys<T>& S, int p, T* buf, con
 #pragma unroll
                 for (int a = 0; a < RA; ++a) c[a] = cb[ti + TR * a];
                 const T my_c = cb[mine], my_u = rb[mine];
-                if (__builtin_expect(__any(rule.small(piv)), 0)) {      // the same for all
-                    flag = 1;
-                    piv = rule.replaced(piv);
-                }
-                const T r = reciprocal(piv);
+                T r = reciprocal(piv);
+                // column / pivot as the column times the reciprocal and its
+                // error, one rounding: an instruction a quotient less
+                const T rerr = nfma(piv, r, T(1)) * r;
+                T l[RA], my_l = mul_add(r, my_c, my_c * rerr);
 #pragma unroll
-                for (int a = 0; a < RA; ++a) {
-                    const T nl = -c[a] * r;
+                for (int a = 0; a < RA; ++a) l[a] = mul_add(r, c[a], c[a] * rerr);
+                if (__builtin_expect(__any(!rule.plain(piv)), 0)) {     // the same for all
+                    if (rule.small(piv)) {
+                        flag = 1;
+                        piv = rule.replaced(piv);
+                    }
+                    r = reciprocal(rule.divisor(piv));
+                    my_l = my_c / piv;
 #pragma unroll
-                    for (int b = 0; b < RB; ++b) x[a][b] = mul_add(nl, u[b], x[a][b]);
+                    for (int a = 0; a < RA; ++a) l[a] = c[a] / piv;
                 }
+#pragma unroll
+                for (int a = 0; a < RA; ++a)
+#pragma unroll
+                    for (int b = 0; b < RB; ++b) x[a][b] = nfma(l[a], u[b], x[a][b]);
                 // position `mine` of the finished row and column
                 if (tid >= k && tid < f.fs) {
-                    S.a[my_row + k] = tid == k ? piv : my_c * r;
+                    S.a[my_row + k] = tid == k ? piv : my_l;
                     S.a[f.fo + k * f.us + tid] = tid == k ? piv : my_u;
                     if (tid == k) S.dinv[f.first + k] = r;
                 }
@@ -440,7 +506,7 @@ __device__ __forceinline__ void forward_quad(const Sys<T>& S, const unsigned sho
     T z = gather(S, f, rr);
     each<0, 16>([&](auto kc) {
         constexpr int k = kc.value;
-        if (TRANS) z = r == k && k < K ? over(z, dg, di) : z;   // U11^T: non-unit
+        if (TRANS) z = r == k && k < K ? quotient(z, dg, di) : z;   // U11^T: non-unit
         const T zk = row_value<k>(z);
         z = r > k && k < K ? nfma(c[k], zk, z) : z;
     });
@@ -468,26 +534,26 @@ __device__ __forceinline__ void backward_quad(const Sys<T>& S, const unsigned sh
     T z = S.y[r < f.K ? f.first + r : int(S.list[f.rows + min(r, f.fs - 1)])];
     each_down<15>([&](auto jc) {
         constexpr int j = jc.value;
-        if (!TRANS) z = r == j && j < f.K ? over(z, dg, di) : z;        // U11: non-unit
+        if (!TRANS) z = r == j && j < f.K ? quotient(z, dg, di) : z;        // U11: non-unit
         const T xj = row_value<j>(z);
         z = r < j && r < f.K && j < fs ? nfma(c[j], xj, z) : z;
     });
     if (have && r < f.K) S.y[f.first + r] = z;
 }
 
-template <bool TRANS, typename T>
+template <bool TRANS, bool EXACT, typename T>
 __device__ __forceinline__ void forward_front(const Sys<T>& S, int p) {
     const int lane = int(threadIdx.x) & 63;
     const Front f = load_front(S, p);
     // the first 64 rows a lane each, the others after the pivots
     const int l0 = min(lane, f.fs - 1), row = f.row(l0);
     T z = gather(S, f, l0);
-#pragma unroll 8
+#pragma unroll (EXACT ? 1 : 8)
     for (int k = 0; k < f.K; ++k) {
         const T c = TRANS ? S.a[f.fo + k * f.us + l0] : S.a[row + k];
         T zk = lane_value(z, k);
         if (TRANS) {                                            // U11^T: non-unit
-            zk = over(zk, S.a[f.fo + k * f.us + k], S.dinv[f.first + k]);
+            zk = over<EXACT>(zk, S.a[f.fo + k * f.us + k], S.dinv[f.first + k]);
             z = lane == k ? zk : z;
         }
         z = lane > k ? nfma(c, zk, z) : z;
@@ -498,7 +564,7 @@ __device__ __forceinline__ void forward_front(const Sys<T>& S, int p) {
         wave_sync();
         for (int l = 64 + lane; l < f.fs; l += 64) {            // K <= 64
             T v = gather(S, f, l);
-#pragma unroll 4
+#pragma unroll (EXACT ? 1 : 4)
             for (int k = 0; k < f.K; ++k)
                 v = nfma(TRANS ? S.a[f.fo + k * f.us + l] : S.a[f.lo + (l - f.K) * f.ls + k], S.y[f.first + k], v);
             S.a[f.wo + l] = v;
@@ -506,7 +572,7 @@ __device__ __forceinline__ void forward_front(const Sys<T>& S, int p) {
     }
 }
 
-template <bool TRANS, typename T>
+template <bool TRANS, bool EXACT, typename T>
 __device__ __forceinline__ void backward_front(const Sys<T>& S, int p) {
     const int lane = int(threadIdx.x) & 63;
     const Front f = load_front(S, p);
@@ -514,15 +580,15 @@ __device__ __forceinline__ void backward_front(const Sys<T>& S, int p) {
     wave_sync();
     const int i = min(lane, f.K - 1);
     T z = S.y[f.first + i];
-#pragma unroll 8
+#pragma unroll (EXACT ? 1 : 8)
     for (int j = f.K; j < f.fs; ++j)
         z = nfma(TRANS ? S.a[f.lo + (j - f.K) * f.ls + i] : S.a[f.fo + i * f.us + j], S.a[f.wo + j], z);
-#pragma unroll 8
+#pragma unroll (EXACT ? 1 : 8)
     for (int k = f.K - 1; k >= 0; --k) {
         const T c = TRANS ? S.a[f.fo + k * f.us + i] : S.a[f.fo + i * f.us + k];
         T xk = lane_value(z, k);
         if (!TRANS) {                                           // U11: non-unit
-            xk = over(xk, S.a[f.fo + k * f.us + k], S.dinv[f.first + k]);
+            xk = over<EXACT>(xk, S.a[f.fo + k * f.us + k], S.dinv[f.first + k]);
             z = lane == k ? xk : z;
         }
         z = lane < k ? nfma(c, xk, z) : z;
@@ -530,8 +596,9 @@ __device__ __forceinline__ void backward_front(const Sys<T>& S, int p) {
     if (lane < f.K) S.y[f.first + lane] = z;
 }
 
-template <bool TRANS, typename T>
-__device__ __forceinline__ void solve_system(const Sys<T>& S) {
+// EXACT: pivots by division, every front on a wave.
+template <bool TRANS, bool EXACT, typename T>
+__device__ __forceinline__ void sweep_system(const Sys<T>& S) {
     const int wave = int(threadIdx.x) >> 6, waves = int(blockDim.x) >> 6;
     for (int s = 0; s < 2 * S.num_levels; ++s) {
         const bool fwd = s < S.num_levels;
@@ -541,15 +608,35 @@ __device__ __forceinline__ void solve_system(const Sys<T>& S) {
         for (int t = wave; t < fronts + quads + shared; t += waves) {
             if (t >= fronts && t < fronts + quads) {
                 const unsigned short* ids = task + fronts + 4 * (t - fronts);
-                if (fwd) forward_quad<TRANS>(S, ids);
-                else backward_quad<TRANS>(S, ids);
+                for (int g = 0; EXACT && g < 4 && ids[g] != 0xffff; ++g) {
+                    if (fwd) forward_front<TRANS, true>(S, ids[g]);
+                    else backward_front<TRANS, true>(S, ids[g]);
+                }
+                if (!EXACT && fwd) forward_quad<TRANS>(S, ids);
+                if (!EXACT && !fwd) backward_quad<TRANS>(S, ids);
             } else {
                 const int p = task[t < fronts ? t : t + 3 * quads];
-                if (fwd) forward_front<TRANS>(S, p);
-                else backward_front<TRANS>(S, p);
+                if (fwd) forward_front<TRANS, EXACT>(S, p);
+                else backward_front<TRANS, EXACT>(S, p);
             }
         }
         __syncthreads();
+    }
+}
+
+// y = A^-1 y (or A^-T y).  A result that is not finite is computed again by
+// division: load() puts the right-hand side into y.
+template <bool TRANS, typename T, class F>
+__device__ __forceinline__ void solve_system(const Sys<T>& S, int n, F load) {
+    load();
+    __syncthreads();
+    sweep_system<TRANS, false>(S);
+    bool finite = true;
+    for (int k = int(threadIdx.x); k < n; k += int(blockDim.x)) finite = finite && __builtin_isfinite(S.y[k]);
+    if (__builtin_expect(__syncthreads_or(!finite), 0)) {
+        load();
+        __syncthreads();
+        sweep_system<TRANS, true>(S);
     }
 }
 
@@ -640,9 +727,9 @@ __global__ __launch_bounds__(NT, 2) void k_sys_solve(SysDevice d, const T* __res
     for (int e = tid; e < d.n; e += NT) S.dinv[e] = in[d.fac + e];
     __syncthreads();
     const unsigned short* perm = S.list + S.o_perm;
-    for (int k = tid; k < d.n; k += NT) S.y[k] = T(rhs[(long long)perm[k] * Bp + b]);
-    __syncthreads();
-    solve_system<TRANS>(S);
+    solve_system<TRANS>(S, d.n, [&] {
+        for (int k = tid; k < d.n; k += NT) S.y[k] = T(rhs[(long long)perm[k] * Bp + b]);
+    });
     for (int k = tid; k < d.n; k += NT) x[(long long)perm[k] * Bp + b] = TX(S.y[k]);
 }
 
@@ -872,9 +959,9 @@ __global__ __launch_bounds__(NT, 2) void k_sys_newton(SysDevice d, NrDevice nr, 
             }
             __syncthreads();
             const unsigned short* perm = S.list + S.o_perm;
-            for (int k = tid; k < d.n; k += NT) S.y[k] = T(n.F[perm[k]]);
-            __syncthreads();
-            solve_system<false>(S);
+            solve_system<false>(S, d.n, [&] {
+                for (int k = tid; k < d.n; k += NT) S.y[k] = T(n.F[perm[k]]);
+            });
             for (int k = tid; k < d.n; k += NT)
                 n.dx[perm[k]] = it > 0 ? n.dx[perm[k]] + double(S.y[k]) : double(S.y[k]);
             __syncthreads();

@@ -7,11 +7,14 @@ hand-over to the level sweeps."""
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import pytest
 import scipy.sparse as sp
 
 import capi
+from test_gpu_lu_capi import LuConfig, _lu_check
 
 pytestmark = pytest.mark.gpu
 
@@ -131,3 +134,77 @@ def test_panel_cap_shapes_the_level_sweeps_only(gpu, cupf, syn):
         V.append(s.solve_batch(g.indptr, g.indices, g.data, g.n_bus, g.n_bus, S, V0, g.pv, g.pq).V_numpy)
     assert sys_plan == {(fronts[64], 5)}
     assert (V[0] == V[1]).all() and (V[0] == V[2]).all()
+
+
+def _factor_solve_unshifted(gpu, A, vals, rhs, precision):
+    """x, x of the transpose and the flags of the inner solver without static pivots."""
+    lib, (B, n) = capi.lib(), rhs.shape
+    cfg = LuConfig()
+    lib.cupf_lu_default_config(ctypes.byref(cfg))
+    cfg.precision, cfg.pivot_strategy, cfg.refine_steps = precision, 0, 0
+    h = ctypes.c_void_p()
+    _lu_check(lib.cupf_lu_create(ctypes.byref(cfg), ctypes.byref(h)))
+    try:
+        rp, ci = A.indptr.astype(np.int32), A.indices.astype(np.int32)
+        _lu_check(lib.cupf_lu_analyze(h, n, A.nnz, ctypes.c_void_p(rp.ctypes.data),
+                                      ctypes.c_void_p(ci.ctypes.data), 0))
+        _lu_check(lib.cupf_lu_setup(h, B))
+        d_vals, d_rhs = gpu.from_numpy(vals).cuda(), gpu.from_numpy(rhs).cuda()
+        d_x, d_xt = gpu.empty_like(d_rhs), gpu.empty_like(d_rhs)
+        p = [ctypes.c_void_p(t.data_ptr()) for t in (d_vals, d_rhs, d_x, d_xt)]
+        _lu_check(lib.cupf_lu_factor(h, p[0], None))
+        _lu_check(lib.cupf_lu_solve(h, p[1], p[2], None))
+        _lu_check(lib.cupf_lu_solve_transpose(h, p[1], p[3], None))
+        flags = np.zeros(B, np.uint8)
+        _lu_check(lib.cupf_lu_singular(h, ctypes.c_void_p(flags.ctypes.data)))
+        return d_x.cpu().numpy(), d_xt.cpu().numpy(), flags
+    finally:
+        _lu_check(lib.cupf_lu_destroy(h))
+
+
+# pivots with a reciprocal that overflows, one that is no normal number, and infinite ones
+ENDS = [(0, 2.0 ** -1030, 2.0 ** 1023), (1, 2.0 ** -130, 2.0 ** 127)]
+
+
+def _ends(tiny, huge, shape):
+    pivots = np.array([huge, -huge, 1.75 * huge, np.inf, -np.inf, tiny, -3 * tiny, 2.0])
+    return pivots[np.random.default_rng(5).integers(0, len(pivots), shape)]
+
+
+@pytest.mark.parametrize("precision,tiny,huge", ENDS)
+def test_quotients_at_the_ends_of_the_range(gpu, precision, tiny, huge):
+    """A diagonal system (fronts of one row), its quotients overflowing and
+    underflowing: exactly what the division gives."""
+    print(f"[sys] quotients precision={precision}", flush=True)
+    T = np.float32 if precision else np.float64
+    top = float(np.finfo(T).max)
+    d = _ends(tiny, huge, (70, 40))
+    b = np.array([1.0, -3.0, tiny, 0.75 * top, top])[np.random.default_rng(6).integers(0, 5, d.shape)]
+    with np.errstate(over="ignore"):
+        want = (b.astype(T) / d.astype(T)).astype(np.float64)
+    assert np.isinf(want).any() and (want == 0).any()
+    x, xt, flags = _factor_solve_unshifted(gpu, sp.identity(40, format="csr"), d, b, precision)
+    assert not flags.any()
+    np.testing.assert_array_equal(x, want)
+    np.testing.assert_array_equal(xt, want)
+
+
+@pytest.mark.parametrize("precision,tiny,huge", ENDS)
+@pytest.mark.parametrize("rows", [12, 24, 40, 90])
+def test_pivots_at_the_ends_of_the_range(gpu, precision, tiny, huge, rows):
+    """The same pivots on the diagonal of a full front of zeros (16 lanes, the
+    workgroup in both its forms): the quotients here are 1, -1, 1/2 and 0, for
+    a zero of the front times an infinite one would be no number by division
+    either."""
+    print(f"[sys] pivots rows={rows} precision={precision}", flush=True)
+    A = sp.csr_matrix(np.ones((rows, rows)))
+    d = _ends(tiny, huge, (70, rows))
+    vals = np.zeros((70, rows * rows))
+    vals[:, ::rows + 1] = d
+    want = np.array([1.0, -1.0, 0.5])[np.random.default_rng(6).integers(0, 3, d.shape)]
+    want[np.isinf(d)] = 0.0
+    b = np.where(np.isinf(d), 1.0, np.where(np.isinf(d), 1.0, d) * want)
+    x, xt, flags = _factor_solve_unshifted(gpu, A, vals, b, precision)
+    assert not flags.any()
+    np.testing.assert_array_equal(x, want)
+    np.testing.assert_array_equal(xt, want)
