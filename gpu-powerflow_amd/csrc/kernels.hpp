@@ -78,8 +78,10 @@ void refine_residual(const int* rp, const int* ci, const int* vmap, const double
                      int Bp, const double* F, const TX* x, double* r, hipStream_t s);
 template <typename TX>
 void axpy_update(const TX* ddx, TX* dx, long long count, hipStream_t s, const int* gate = nullptr);
-// out[0 .. sum_squares_parts) = sums of v[i * Bp + b]^2 over blocks of rows and
-// scenarios b < B, in a fixed order; at most dim * Bp / 256 + 1 parts.
+// The sum of v[i * Bp + b]^2 over rows and scenarios b < B in
+// sum_squares_parts = ceil(dim / 64) * Bp / 64 parts of three: (out[0] + out[1])
+// * 2^(2 out[2]), out[1] at most a rounding of out[0] (no number where out[0] is
+// infinite); in a fixed order.
 int sum_squares_parts(int dim, int Bp);
 void sum_squares(const double* v, int dim, int B, int Bp, double* out, hipStream_t s);
 // max over scenarios b < B of normF[b] -> out[0]

@@ -1143,19 +1143,23 @@ void NewtonSolver::solve_adjoint(const double* grad_va, int64_t grad_va_stride,
     if (options.check_residual) {
         m.lu.residual<double>(m.J.as<double>(), m.g.as<double>(), m.lam.as<double>(), m.lu.res(),
                               true, m.Bp, m.s);
-        // sums of squares per block of rows on the device, their total here
+        // sums of squares per block of rows on the device, their total here; the
+        // solve's scratch vector (at least 64 * dim FP32 values) holds them
         const int parts = kern::sum_squares_parts(m.js.dim, m.Bp);
-        std::vector<double> sums(2 * size_t(parts));
-        kern::sum_squares(m.lu.res(), m.js.dim, B, m.Bp, m.stage_c.as<double>(), m.s);
-        kern::sum_squares(m.g.as<double>(), m.js.dim, B, m.Bp, m.stage_c.as<double>() + parts, m.s);
-        CUPF_HIP(hipMemcpyAsync(sums.data(), m.stage_c.get(), sums.size() * sizeof(double),
+        std::vector<double> sums(6 * size_t(parts));
+        kern::sum_squares(m.lu.res(), m.js.dim, B, m.Bp, m.ddx.as<double>(), m.s);
+        kern::sum_squares(m.g.as<double>(), m.js.dim, B, m.Bp, m.ddx.as<double>() + 3 * parts, m.s);
+        CUPF_HIP(hipMemcpyAsync(sums.data(), m.ddx.get(), sums.size() * sizeof(double),
                                 hipMemcpyDeviceToHost, m.s));
         CUPF_HIP(hipStreamSynchronize(m.s));
-        long double rr = 0, gg = 0;
-        for (int i = 0; i < parts; ++i) {
-            rr += sums[size_t(i)];
-            gg += sums[size_t(parts + i)];
-        }
+        auto total = [&](const double* p) {
+            long double t = 0;
+            for (int i = 0; i < parts; ++i, p += 3)
+                t += std::isfinite(p[0]) ? std::ldexp((long double)p[0] + p[1], 2 * int(p[2]))
+                                         : (long double)p[0];
+            return t;
+        };
+        const long double rr = total(sums.data()), gg = total(sums.data() + 3 * size_t(parts));
         const long double den =
             std::max(std::sqrt(std::max(gg, (long double)1e-60)), (long double)1e-30);
         result.jt_residual_norm = double(std::sqrt(rr) / den);

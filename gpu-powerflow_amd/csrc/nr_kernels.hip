@@ -302,26 +302,61 @@ __global__ __launch_bounds__(kBlock) void k_axpy(const TX* __restrict__ a, TX* _
     if (i < count) x[i] += a[i];
 }
 
-// Bound by the read of v; a block sums kSumRows rows of 64 scenarios.
+// Bound by the read of v; a block sums kSumRows rows of 64 scenarios.  The
+// squares are summed in two doubles (hi + lo), exactly but for some 2^-100, of
+// values scaled by the block's largest exponent, so that no square over- or
+// underflows that counts.
 constexpr int kSumRows = 64;
+__device__ __forceinline__ void add_exact(double& hi, double& lo, double v, double rest) {
+    const double s = hi + v, t = s - hi;
+    lo += ((hi - (s - t)) + (v - t)) + rest;
+    hi = s;
+}
 __global__ __launch_bounds__(kBlock) void k_sum_squares(const double* __restrict__ v, int dim, int B,
                                                         int Bp, double* __restrict__ out) {
+    constexpr int kEach = kSumRows / kWaves;
     const int lane = threadIdx.x & (kLanes - 1), w = threadIdx.x / kLanes;
     const int b = blockIdx.y * kLanes + lane;
-    double acc = 0.0;
-    if (b < B)
-        for (int i = blockIdx.x * kSumRows + w; i < min(dim, int(blockIdx.x + 1) * kSumRows); i += kWaves) {
-            const double x = v[(long long)i * Bp + b];
-            acc = fma(x, x, acc);
-        }
-    __shared__ double red[kBlock];
-    red[threadIdx.x] = acc;
+    __shared__ double red[2][kBlock];
+    double x[kEach], m = 0.0;
+#pragma unroll
+    for (int i = 0; i < kEach; ++i) {
+        const int r = blockIdx.x * kSumRows + w + kWaves * i;
+        x[i] = b < B && r < dim ? v[(long long)r * Bp + b] : 0.0;
+        m = fmax(m, fabs(x[i]));
+    }
+    red[0][threadIdx.x] = m;
     __syncthreads();
     for (int s = kBlock / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
+        if (threadIdx.x < s) red[0][threadIdx.x] = fmax(red[0][threadIdx.x], red[0][threadIdx.x + s]);
         __syncthreads();
     }
-    if (threadIdx.x == 0) out[blockIdx.y * gridDim.x + blockIdx.x] = red[0];
+    m = red[0][0];
+    const int e = m > 0.0 && isfinite(m) ? ilogb(m) : 0;
+    __syncthreads();
+    double hi = 0.0, lo = 0.0;
+#pragma unroll
+    for (int i = 0; i < kEach; ++i) {
+        const double y = ldexp(x[i], -e), p = y * y;
+        add_exact(hi, lo, p, fma(y, y, -p));
+    }
+    red[0][threadIdx.x] = hi;
+    red[1][threadIdx.x] = lo;
+    __syncthreads();
+    for (int s = kBlock / 2; s > 0; s >>= 1) {
+        if (threadIdx.x < s) {
+            add_exact(hi, lo, red[0][threadIdx.x + s], red[1][threadIdx.x + s]);
+            red[0][threadIdx.x] = hi;
+            red[1][threadIdx.x] = lo;
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        double* o = out + 3 * (blockIdx.y * gridDim.x + blockIdx.x);
+        o[0] = hi;
+        o[1] = lo;
+        o[2] = e;
+    }
 }
 
 __global__ __launch_bounds__(kBlock) void k_batch_max(const double* __restrict__ v, int B,

@@ -276,3 +276,37 @@ def test_torch_dtype_rule(gpu, cupf, syn):
     zb = torch.zeros(g.n_bus, device=dev, dtype=torch.float32)
     with pytest.raises(ValueError, match="float64"):
         s.solve_torch(zb, zb, z, z, zb, zb + 1, torch.empty_like(z), torch.empty_like(z))
+
+
+@pytest.mark.parametrize("n,B", [(2, 1), (2, 65), (118, 1), (118, 65), (300, 130)])
+def test_residual_norm_at_every_scale_and_over_its_parts(gpu, cupf, syn, n, B):
+    """jt_residual_norm = ||g - J^T lambda|| / ||g|| over the batch.  FP64 is
+    exact under powers of two, so it is the same to the bit where the squares
+    leave the range of a double; and the batch's is made up of its parts', found
+    by zeroing the gradients of the other scenarios (1e-13: a square root, a
+    division and their rounding to double)."""
+    print(f"[adjoint] residual norm n={n} B={B}", flush=True)
+    g = syn.make_grid(n, max(n - 1, int(1.55 * n)) if n > 2 else 1, int(0.15 * n), seed=n,
+                      load_scale=min(0.25, 100.0 / n))
+    s = make_solver(cupf, g)
+    so = cupf.SolveOptions()
+    so.prepare_adjoint_cache = True
+    s.solve_batch(g.indptr, g.indices, g.data, n, n, g.sbus_scaled(syn.load_factors(B, n, 0.7, 1.3, 1)),
+                  g.flat_start(B), g.pv, g.pq, cupf.NRConfig(), so)
+    rng = np.random.default_rng(2)
+    gva, gvm = rng.standard_normal((2, B, n))
+
+    def norm(scale=1.0, of=slice(None)):
+        m = np.zeros((B, 1))
+        m[of] = scale
+        return s.solve_adjoint(m * gva, m * gvm, g.pv, g.pq, cupf.AdjointOptions()).jt_residual_norm
+
+    whole = norm()
+    assert 0 < whole <= 1e-12 or n == 2
+    for k in (300, 530, 900):
+        assert norm(2.0 ** k) == whole, k
+    pvpq = np.concatenate([g.pv, g.pq])
+    gg = (gva[:, pvpq].astype(np.longdouble) ** 2).sum(1) + (gvm[:, g.pq].astype(np.longdouble) ** 2).sum(1)
+    parts = [slice(0, B // 2), slice(B // 2, B - 1), slice(B - 1, B)]
+    rr = sum(np.longdouble(norm(of=p)) ** 2 * gg[p].sum() for p in parts)
+    assert abs(np.sqrt(rr / gg.sum()) - whole) <= 1e-13 * whole
