@@ -148,7 +148,9 @@ struct NewtonSolver::Impl {
     int pred_steps[2] = {0, 0};       // steps the last device-run loop of each kind took
     unsigned pred_pattern[2] = {0, 0};  // and which of them wanted refinement
     unsigned long long buf_gen = 1;   // bumped whenever a device buffer the step uses moves
-    bool graph_warm = false;          // first loop eager (first-use kernel attributes)
+    // the loops that ran eagerly, so that no kernel's first use (its attributes,
+    // its code's load) falls into a capture: level sweeps, one-workgroup kernels
+    bool graph_warm[2] = {false, false};
     const void* head_warm = nullptr;  // the last head run eagerly (its first use likewise)
     bool capturing = false;
     bool count_factor = true;         // factor() counts itself (not inside the device loop)
@@ -460,9 +462,8 @@ struct NewtonSolver::Impl {
 
     // Device-run NR loop (the captured form of the reference's graph
     // iteration, graph_iteration.hpp:85-146): the residual at the initial V
-    // and at most limit - 1 steps; completed = 1 + steps.  The first loop on
-    // a solver runs the same launches eagerly (first-use kernel attributes
-    // are set outside capture).
+    // and at most limit - 1 steps; completed = 1 + steps.  The first loop of
+    // either kind on a solver runs the same launches eagerly.
     int run_nr_device(const NRConfig& cfg, bool tolerant, int limit,
                       const std::function<void()>& head, const void* head_id,
                       unsigned long long head_gen) {
@@ -474,14 +475,15 @@ struct NewtonSolver::Impl {
         const int ti = tolerant ? 1 : 0;
         int c[5] = {0, 0, 0, 0, 0};
         double m = 0.0;
-        if (!graph_warm || (head_id && head_id != head_warm)) {
+        bool& ran = graph_warm[sys_loop() ? 1 : 0];
+        if (!ran || (head_id && head_id != head_warm)) {
             loop_head(head, cfg, tolerant, limit);
             read_control(c, m);
             while (!c[0]) {
                 loop_step(cfg, tolerant, limit, c[1] == 0);
                 read_control(c, m);
             }
-            graph_warm = true;
+            ran = true;
             if (head_id) head_warm = head_id;
         } else {
             const int steps = std::min(pred_steps[ti], limit - 1);
@@ -927,7 +929,7 @@ void NewtonSolver::initialize(const YbusView& ybus, const int32_t* pv, int32_t n
     for (DeviceBuffer* b : {&m.warm_v0, &m.warm_s, &m.warm_r, &m.warm_o, &m.warm_y}) b->release();
     m.warm_cap = 0;
     m.drop_graph();
-    m.graph_warm = false;
+    m.graph_warm[0] = m.graph_warm[1] = false;
     m.head_warm = nullptr;
     ++m.buf_gen;
     m.st = NewtonSolverStats{};

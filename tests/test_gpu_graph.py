@@ -136,3 +136,23 @@ def test_batch_one_graph(gpu, cupf, syn, compute):
         V0 = g.flat_start(1)
         _check_same(eager.solve_batch(*args, S, V0, g.pv, g.pq),
                     graph.solve_batch(*args, S, V0, g.pv, g.pq))
+
+
+def test_both_kinds_of_loop_run_eagerly_before_their_capture(gpu, cupf, syn):
+    """70 scenarios of 30 buses run the one-workgroup kernels, 2,049 the level
+    sweeps: the first solve of either kind launches no graph, so no kernel is
+    used for the first time inside a capture; every later one is one launch,
+    and all equal the eager solver's."""
+    g = syn.make_grid(30, 46, 4, seed=30, load_scale=0.25)
+    eager = _solver(cupf, g, "FP64", False)
+    graph = _solver(cupf, g, "FP64", True)
+    S = g.sbus_scaled(syn.load_factors(2049, 30, 0.7, 1.3, 6))
+    V0 = g.flat_start(2049)
+    args = (g.indptr, g.indices, g.data, 30, 30)
+    for B, launches in [(70, 0), (2049, 0), (2049, 1), (70, 1), (2049, 1)]:
+        print(f"[graph] B={B}", flush=True)
+        re = eager.solve_batch(*args, S[:B], V0[:B], g.pv, g.pq)
+        before = graph.stats()["graph_launches"]
+        rg = graph.solve_batch(*args, S[:B], V0[:B], g.pv, g.pq)
+        assert graph.stats()["graph_launches"] - before == launches
+        _check_same(re, rg)
