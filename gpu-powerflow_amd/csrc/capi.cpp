@@ -484,6 +484,13 @@ int cupf_solver_debug_pattern(cupf_solver* solver, int32_t* row_ptr, int32_t* co
     return guarded([&] { solver_of(solver).debug_pattern(row_ptr, col_idx, perm); });
 }
 
+int cupf_solver_debug_captures(cupf_solver* solver, int64_t* out) {
+    return guarded([&] {
+        if (!out) throw std::invalid_argument("null argument");
+        *out = solver_of(solver).debug_captures();
+    });
+}
+
 int cupf_solver_debug_plan(cupf_solver* solver, int32_t* out4) {
     return guarded([&] {
         if (!out4) throw std::invalid_argument("null argument");

@@ -147,6 +147,7 @@ struct NewtonSolver::Impl {
     GraphKey step_keys[2][2];
     int pred_steps[2] = {0, 0};       // steps the last device-run loop of each kind took
     unsigned pred_pattern[2] = {0, 0};  // and which of them wanted refinement
+    int64_t captures = 0;             // graphs captured since the solver was made
     unsigned long long buf_gen = 1;   // bumped whenever a device buffer the step uses moves
     // the loops that ran eagerly, so that no kernel's first use (its attributes,
     // its code's load) falls into a capture: level sweeps, one-workgroup kernels
@@ -433,6 +434,7 @@ struct NewtonSolver::Impl {
     // Capture body() on the private stream into an executable graph.
     hipGraphExec_t capture(const std::function<void()>& body) {
         const hipStream_t call = s;
+        ++captures;
         s = own;
         capturing = true;
         hipGraph_t g = nullptr;
@@ -486,9 +488,13 @@ struct NewtonSolver::Impl {
             ran = true;
             if (head_id) head_warm = head_id;
         } else {
-            const int steps = std::min(pred_steps[ti], limit - 1);
+            // the one-workgroup launches decide on the refinement themselves, and
+            // one scenario's first launch runs the whole loop
+            const bool sys = sys_loop();
+            const int steps = sys && B == 1 ? 0 : std::min(pred_steps[ti], limit - 1);
             const unsigned pattern =
-                refine > 0 ? pred_pattern[ti] & (steps >= 32 ? ~0u : (1u << steps) - 1u) : 0u;
+                refine > 0 && !sys ? pred_pattern[ti] & (steps >= 32 ? ~0u : (1u << steps) - 1u) : 0u;
+            if (head) seed_in_loop = sys;           // as the head leaves it
             GraphKey key{B, Bp, ti, refine, limit, steps, pattern, cfg.tolerance, nr.yb, head_id,
                          buf_gen, head_gen, seed_in_loop};
             if (!solve_graphs[ti] || !(key == solve_keys[ti])) {
@@ -496,8 +502,7 @@ struct NewtonSolver::Impl {
                 solve_graphs[ti] = nullptr;
                 solve_graphs[ti] = capture([&] {
                     loop_head(head, cfg, tolerant, limit);
-                    // one scenario's first launch runs the whole loop
-                    for (int k = 0; k < (sys_loop() && B == 1 ? 0 : steps); ++k)
+                    for (int k = 0; k < steps; ++k)
                         loop_step(cfg, tolerant, limit, k < 32 && ((pattern >> k) & 1u));
                 });
                 solve_keys[ti] = key;
@@ -508,8 +513,9 @@ struct NewtonSolver::Impl {
             key.steps = 1;
             key.head = nullptr;
             key.head_gen = 0;
+            key.seed = false;                       // the first launch's
             while (!c[0]) {
-                const int ri = c[1] == 0 && refine > 0 ? 1 : 0;
+                const int ri = c[1] == 0 && refine > 0 && !sys ? 1 : 0;
                 key.pattern = unsigned(ri);
                 hipGraphExec_t& sg = step_graphs[ti][ri];
                 if (!sg || !(key == step_keys[ti][ri])) {
@@ -1391,6 +1397,8 @@ void NewtonSolver::debug_pattern(int32_t* row_ptr, int32_t* col_idx, int32_t* pe
     std::copy(m.js.col_idx.begin(), m.js.col_idx.end(), col_idx);
     std::copy(m.lu.plan().perm.begin(), m.lu.plan().perm.end(), perm);
 }
+
+int64_t NewtonSolver::debug_captures() const { return impl_->captures; }
 
 void NewtonSolver::debug_plan(int32_t* out4) const {
     const Impl& m = *impl_;

@@ -125,6 +125,8 @@ public:
     // Fronts and levels of the level sweeps' plan, then of the one-workgroup
     // plan (0, 0: the system does not qualify).
     void debug_plan(int32_t* out4) const;
+    // Graphs captured since the solver was made (use_cuda_graph).
+    int64_t debug_captures() const;
 
 private:
     struct Impl;

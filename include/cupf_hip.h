@@ -237,6 +237,8 @@ int cupf_solver_debug_pattern(cupf_solver* solver, int32_t* row_ptr, int32_t* co
 /* fronts and levels of the level sweeps' plan, then of the one-workgroup plan
  * (0, 0: the system does not qualify for it) */
 int cupf_solver_debug_plan(cupf_solver* solver, int32_t out4[4]);
+/* graphs captured since the solver was made (use_cuda_graph) */
+int cupf_solver_debug_captures(cupf_solver* solver, int64_t* out);
 
 /* ---- Host analysis (no GPU needed) ------------------------------------ */
 /* Jacobian pattern + scatter maps; the reference's make_jacobian_indexing /

@@ -179,3 +179,9 @@ def debug_plan(handle):
     out = np.zeros(4, np.int32)
     check(lib().cupf_solver_debug_plan(_h(handle), _p(out)))
     return dict(zip(("fronts", "levels", "sys_fronts", "sys_levels"), out.tolist()))
+
+
+def debug_captures(handle):
+    out = ctypes.c_int64()
+    check(lib().cupf_solver_debug_captures(_h(handle), ctypes.byref(out)))
+    return out.value

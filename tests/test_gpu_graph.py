@@ -21,6 +21,8 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
+import capi
+
 pytestmark = pytest.mark.gpu
 
 
@@ -156,3 +158,47 @@ def test_both_kinds_of_loop_run_eagerly_before_their_capture(gpu, cupf, syn):
         rg = graph.solve_batch(*args, S[:B], V0[:B], g.pv, g.pq)
         assert graph.stats()["graph_launches"] - before == launches
         _check_same(re, rg)
+
+
+def test_small_grids_keep_their_graphs(gpu, cupf, syn):
+    """The one-workgroup launches do not depend on the refinement pattern, nor,
+    for one scenario, on the step count: starts that take different steps, and
+    torch forwards between warm-started solves, reuse the graphs there are."""
+    torch = gpu
+    g = syn.workload_grid("case118")
+    n = g.n_bus
+    args = (g.indptr, g.indices, g.data, n, n)
+    eager, graph = (_solver(cupf, g, "Mixed", on) for on in (False, True))
+    S, V0 = g.sbus_scaled(syn.load_factors(256, n, 0.7, 1.3, 8)), g.flat_start(256)
+    V = eager.solve_batch(*args, S, V0, g.pv, g.pq).V_numpy
+
+    def near(scale):
+        v = V * np.exp(1j * scale * np.random.default_rng(1).standard_normal(V.shape))
+        v[:, g.slack] = V0[:, g.slack]
+        return v
+
+    def solve(B, start):
+        _check_same(eager.solve_batch(*args, S[:B], start[:B], g.pv, g.pq),
+                    graph.solve_batch(*args, S[:B], start[:B], g.pv, g.pq))
+        return capi.debug_captures(graph.handle)
+
+    starts = [V0, near(1e-4), near(1e-2), near(1e-7), V0]
+    assert [solve(1, v) for v in starts] == [0, 1, 1, 1, 1]
+    assert len({int(eager.solve_batch(*args, S[:1], v[:1], g.pv, g.pq).iterations_numpy[0]) for v in starts}) > 2
+
+    mlp, _ = cupf.train_warm_start(eager, torch.from_numpy(S).cuda(), torch.from_numpy(V0).cuda(), g.pv, g.pq,
+                                   hidden=64, depth=2, epochs=3, batch=64, lr=2e-3, seed=0, skip=False)
+    graph.set_warm_start(mlp, 10)
+    t = [torch.from_numpy(np.ascontiguousarray(v, np.float32)).cuda()
+         for v in (g.p_gen, np.zeros(n), np.tile(g.p_load, (256, 1)), np.tile(g.q_load, (256, 1)),
+                   np.angle(V0[0]), np.abs(V0[0]))]
+    new = []
+    for call in range(4):
+        print(f"[graph] warm call {call}", flush=True)
+        before = capi.debug_captures(graph.handle)
+        assert graph.solve_batch(*args, S, V0, g.pv, g.pq).converged_numpy.all()
+        assert graph.stats()["last_warm_fallbacks"] == 0
+        new.append(capi.debug_captures(graph.handle) - before)
+        if call == 1:
+            cupf.solve(t[2], t[3], graph, sbus_base_re=t[0], sbus_base_im=t[1], v0_va=t[4], v0_vm=t[5])
+    assert new == [0, 1, 0, 0]         # eager, captured, then launched
