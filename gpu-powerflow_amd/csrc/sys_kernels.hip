@@ -120,10 +120,9 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Pivot row and column buffers: 128 elements a wave for eight waves, or four
-// times the rows of a shared front.
-constexpr int kSysBuf = 1024;
-static_assert(kSysBuf >= 4 * kSysMaxRows, "a shared front's buffers");
+// Pivot row and column buffers: a share for each of eight waves, or all of
+// them for a shared front.
+constexpr int kWaveBuf = 128, kSysBuf = 8 * kWaveBuf;
 
 // The tables and arrays of one system in LDS.  `a` holds the factors at 0 and
 // the scratch region (contribution blocks, then work vectors) at scr.
@@ -354,6 +353,7 @@ __device__ __forceinline__ void factor_quad(const Sys<T>& S, const unsigned shor
 template <typename T, int RA, int RB, int TR, int TC, bool ALL>
 __device__ __forceinline__ void factor_front(const Sys<T>& S, int p, T* buf, const PivotRule<T>& rule, int& flag) {
     constexpr int kRows = TR * RA, kCols = TC * RB;             // buf: [2][kRows + kCols]
+    static_assert(2 * (kRows + kCols) <= (ALL ? kSysBuf : kWaveBuf), "the team's buffers");
     const int tid = ALL ? int(threadIdx.x) : int(threadIdx.x) & 63;
     const int ti = tid / TC, tj = tid % TC;
     auto sync = [] {
@@ -454,7 +454,7 @@ __device__ __forceinline__ void factor_system(const Sys<T>& S, double eps, int s
         const int quads = lv[1], fronts = lv[2], shared = lv[3];
         for (int t = wave; t < fronts + quads; t += waves) {
             if (t >= fronts) factor_quad(S, task + fronts + 4 * (t - fronts), rule, flag);
-            else factor_front<T, 4, 4, 8, 8, false>(S, task[t], S.buf + wave * 128, rule, flag);
+            else factor_front<T, 4, 4, 8, 8, false>(S, task[t], S.buf + wave * kWaveBuf, rule, flag);
         }
         __syncthreads();
         for (int t = 0; t < shared; ++t) {
