@@ -386,10 +386,17 @@ Symbolic analyze_symbolic(int n, const int* rp, const int* ci, const std::vector
     fill_pattern(n, s.sym_cp.data(), s.sym_ri.data(), s.parent, s.Lp, s.Li);
     s.colcount.resize(n);
     for (int j = 0; j < n; ++j) s.colcount[j] = s.Lp[j + 1] - s.Lp[j];
+    cut_panels(s, cap);
+    return s;
+}
 
+void cut_panels(Symbolic& s, int cap) {
+    const int n = s.n;
     // Relaxed panels: grow along parent[j] == j + 1 chains up to `cap`
     // columns (supernode.cpp:104-141).
     s.cap = cap < 1 ? 1 : cap;
+    s.num_panels = 0;
+    for (std::vector<int>* v : {&s.panel_first, &s.panel_ncols, &s.panel_width, &s.front_rows}) v->clear();
     s.panel_of.assign(n, -1);
     for (int j = 0; j < n;) {
         const int start = j;
@@ -444,7 +451,6 @@ Symbolic analyze_symbolic(int n, const int* rp, const int* ci, const std::vector
             if (it != s.front_rows.data() + pe && *it == r) s.asm_idx[a] = int(it - s.front_rows.data());
         }
     }
-    return s;
 }
 
 // ===========================================================================

@@ -73,6 +73,8 @@ std::vector<int> order_jacobian(const JacobianStructure& js);
 std::vector<int> order_matrix(int n, const int* rp, const int* ci);
 
 // Full symbolic pipeline for a given order (no reordering is done here).
+// cut_panels() cuts an analysed matrix into panels and fronts at another cap.
+void cut_panels(Symbolic& s, int cap);
 Symbolic analyze_symbolic(int n, const int* rp, const int* ci, const std::vector<int>& perm,
                           int cap);
 

@@ -171,7 +171,7 @@ void BatchedLU::analyze(int n, const int* rp, const int* ci, const std::vector<i
     lu.gat_ptr = d_gptr.as<int>(); lu.gat_src = d_gsrc.as<int>(); lu.rhs_idx = d_ridx.as<int>();
 
     find_chains(s);
-    find_sys(opt.n_bus, rp, ci, perm, s);
+    find_sys(opt.n_bus, rp, ci, s);
 
     // The timed dense stage is one kernel: the tile kernel when any level
     // takes it, else the row-block Schur kernel, else the tier-2 LU groups.
@@ -263,11 +263,10 @@ void BatchedLU::analyze(int n, const int* rp, const int* ci, const std::vector<i
 // against 1.16.  The line lies where every measured shape gains.
 constexpr int kSysPerCu = 1024, kSysEver = 2048;
 
-void BatchedLU::find_sys(int n_bus, const int* rp, const int* ci, const std::vector<int>& perm,
-                         hipStream_t s) {
+void BatchedLU::find_sys(int n_bus, const int* rp, const int* ci, hipStream_t s) {
     sys_ = SysPlan{};
     sys_dev_ = kern::SysDevice{};
-    sys_ = find_sys_plan(plan_, opt_.cap, rp, ci, perm, kern::kSysLdsMax / front_bytes());
+    sys_ = find_sys_plan(plan_, sym_, rp, ci, kern::kSysLdsMax / front_bytes());
     if (!sys_.ok) return;
     sys_lds_ = kern::sys_lds_bytes(sys_, int(front_bytes()), 0);
     if (kern::sys_lds_bytes(sys_, int(front_bytes()), n_bus) > kern::kSysLdsMax) {

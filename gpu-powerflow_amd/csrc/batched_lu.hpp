@@ -143,7 +143,7 @@ private:
     bool tile_schur(int level) const;
     size_t uinv_elems(int Bp) const;
     void find_chains(hipStream_t s);
-    void find_sys(int n_bus, const int* rp, const int* ci, const std::vector<int>& perm, hipStream_t s);
+    void find_sys(int n_bus, const int* rp, const int* ci, hipStream_t s);
     int scenarios(int Bp) const;
     bool sys_batch(int Bp) const { return sys_.ok && Bp <= sys_most_; }
     void split_tier1();

@@ -576,7 +576,7 @@ int cupf_plan_sys(int32_t n, const int32_t* row_ptr, const int32_t* col_idx, con
         const cupf::Symbolic s = cupf::analyze_symbolic(n, row_ptr, col_idx, pv, cap);
         const cupf::LuPlan p = cupf::lower_plan(s, n, row_ptr, col_idx);
         const cupf::SysPlan q =
-            cupf::find_sys_plan(p, cap, row_ptr, col_idx, pv, cupf::kern::kSysLdsMax / size_t(elem));
+            cupf::find_sys_plan(p, s, row_ptr, col_idx, cupf::kern::kSysLdsMax / size_t(elem));
         out3[0] = q.ok ? q.num_fronts : 0;
         out3[1] = q.ok ? q.num_levels : 0;
         out3[2] = q.ok ? q.fac + q.scratch : 0;

@@ -6,6 +6,9 @@
 namespace cupf {
 
 namespace {
+// LDS elements of a front's factors.
+long long factor_elems(int fs, int K) { return (long long)K * (fs | 1) + (long long)(fs - K) * (K | 1); }
+
 // A front is shared by the whole workgroup when its level has too few fronts
 // to occupy the waves, or when it exceeds a wave's registers.
 constexpr int kAloneFronts = 2;
@@ -53,9 +56,8 @@ SysPlan make_sys_plan(const LuPlan& P, size_t most_elems) {
     // sizes first: a system that is too large costs one pass over its fronts,
     // and the allocation below (fronts squared) ends where the blocks no longer fit
     for (int p = 0; p < F; ++p) {
-        const int fs = P.fsz[p], K = P.nc[p], uc = fs - K;
-        fac += (long long)K * (fs | 1) + (long long)uc * (K | 1);
-        work += fs;
+        fac += factor_elems(P.fsz[p], P.nc[p]);
+        work += P.fsz[p];
     }
     if (size_t(fac + work) > most_elems) return S;
     for (int p : order) {
@@ -66,11 +68,11 @@ SysPlan make_sys_plan(const LuPlan& P, size_t most_elems) {
     }
     fac = work = 0;
     for (int p = 0; p < F; ++p) {
-        const int fs = P.fsz[p], K = P.nc[p], uc = fs - K;
+        const int fs = P.fsz[p], K = P.nc[p];
         SysFront& f = fr[size_t(p)];
         f.fo = int(fac);
         f.wo = int(work);
-        fac += (long long)K * (fs | 1) + (long long)uc * (K | 1);
+        fac += factor_elems(fs, K);
         work += fs;
         f.size = fs | K << 16;
         f.first = P.front_rows[P.front_ptr[p]];
@@ -206,14 +208,19 @@ SysPlan make_sys_plan(const LuPlan& P, size_t most_elems) {
     return S;
 }
 
-SysPlan find_sys_plan(const LuPlan& P, int cap, const int* rp, const int* ci, const std::vector<int>& perm,
-                      size_t most_elems) {
+SysPlan find_sys_plan(const LuPlan& P, const Symbolic& sym, const int* rp, const int* ci, size_t most_elems) {
     // Entries of L and U off the diagonal: the least elements of the factors at
     // any cap, known without another analysis.  Fronts only grow with the cap,
     // so those of a narrower plan tell too.
-    if (size_t(2 * (P.lnz - P.n)) > most_elems || (cap <= kSysCap && P.max_fsz > kSysMaxRows)) return SysPlan{};
-    if (cap == kSysCap) return make_sys_plan(P, most_elems);
-    return make_sys_plan(lower_plan(analyze_symbolic(P.n, rp, ci, perm, kSysCap), P.n, rp, ci), most_elems);
+    if (size_t(2 * (P.lnz - P.n)) > most_elems || (sym.cap <= kSysCap && P.max_fsz > kSysMaxRows))
+        return SysPlan{};
+    if (sym.cap == kSysCap) return make_sys_plan(P, most_elems);
+    Symbolic at = sym;
+    cut_panels(at, kSysCap);
+    long long fac = 0;
+    for (int p = 0; p < at.num_panels; ++p) fac += factor_elems(at.front_ptr[p + 1] - at.front_ptr[p], at.panel_ncols[p]);
+    if (size_t(fac) > most_elems) return SysPlan{};
+    return make_sys_plan(lower_plan(at, P.n, rp, ci), most_elems);
 }
 
 }  // namespace cupf

@@ -72,8 +72,7 @@ constexpr int kSysCap = 64;
 SysPlan make_sys_plan(const LuPlan& P, size_t most_elems);
 
 // The one-workgroup plan (ok false: the system does not qualify) of the pattern
-// rp/ci in the order perm, whose plan at the caller's cap is P.
-SysPlan find_sys_plan(const LuPlan& P, int cap, const int* rp, const int* ci, const std::vector<int>& perm,
-                      size_t most_elems);
+// rp/ci, whose analysis and plan at the caller's cap are sym and P.
+SysPlan find_sys_plan(const LuPlan& P, const Symbolic& sym, const int* rp, const int* ci, size_t most_elems);
 
 }  // namespace cupf
