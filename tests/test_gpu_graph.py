@@ -13,7 +13,9 @@ batches it takes the same steps as the eager loop and the results are
 bit-identical.  Covered: several solves in a row (a new batch size
 recaptures), a prediction above the steps a batch needs (the gated steps do
 nothing), below it (continuation steps), the refinement decided on the device
-(Mixed), a warm-started solve in one launch, and the batch-1 kernels.
+(Mixed), a warm-started solve in one launch, and batch 1; each on a grid that
+runs the one-workgroup kernels (118 buses) and on one that runs the level
+sweeps (400 buses).
 """
 
 from __future__ import annotations
@@ -38,9 +40,22 @@ def _solver(cupf, g, compute, graph, refine=1):
     return s
 
 
+@pytest.fixture(params=[118, 400])
+def grid(request, syn):
+    if request.param == 118:
+        return syn.workload_grid("case118")
+    return syn.make_grid(400, 620, 60, seed=400, load_scale=0.25)
+
+
+def test_the_grids_run_either_kind_of_loop(gpu, cupf, grid):
+    for compute in ("Mixed", "FP64"):
+        s = _solver(cupf, grid, compute, False)      # the handle is the solver's
+        assert (capi.debug_plan(s.handle)["sys_fronts"] > 0) == (grid.n_bus == 118)
+
+
 @pytest.mark.parametrize("compute", ["Mixed", "FP64"])
-def test_graph_step_matches_eager(gpu, cupf, syn, compute):
-    g = syn.workload_grid("case118")
+def test_graph_step_matches_eager(gpu, cupf, syn, grid, compute):
+    g = grid
     eager = _solver(cupf, g, compute, False)
     graph = _solver(cupf, g, compute, True)
     for call, (B, seed) in enumerate([(70, 3), (70, 4), (70, 3), (33, 5), (70, 6)]):
@@ -64,12 +79,12 @@ def _check_same(re, rg):
 
 
 @pytest.mark.parametrize("compute", ["Mixed", "FP64"])
-def test_gated_steps_over_and_under_the_prediction(gpu, cupf, syn, compute):
+def test_gated_steps_over_and_under_the_prediction(gpu, cupf, syn, grid, compute):
     """A flat start (6 or so iterations) teaches the prediction; a start at a
     near-solution then needs fewer steps (the captured solve runs gated
     no-op steps after convergence), and a flat start again needs more than
     that prediction (continuation steps); each equals the eager solver."""
-    g = syn.workload_grid("case118")
+    g = grid
     eager = _solver(cupf, g, compute, False)
     graph = _solver(cupf, g, compute, True)
     B = 70
@@ -93,13 +108,13 @@ def test_gated_steps_over_and_under_the_prediction(gpu, cupf, syn, compute):
     assert graph.stats()["factorizations"] == eager.stats()["factorizations"] - eager_before
 
 
-def test_warm_start_inside_the_captured_solve(gpu, cupf, syn):
+def test_warm_start_inside_the_captured_solve(gpu, cupf, syn, grid):
     """A warm-started solve: inference, the tolerant warm pass and the stop
     tests in one captured launch once the step count is known; V,
     iterations and fallbacks equal the eager solver's with the same
     network."""
     torch = gpu
-    g = syn.workload_grid("case118")
+    g = grid
     eager = _solver(cupf, g, "Mixed", False)
     graph = _solver(cupf, g, "Mixed", True)
     St = torch.from_numpy(g.sbus_scaled(syn.load_factors(2048, g.n_bus, 0.6, 1.4, seed=2))).cuda()
@@ -127,9 +142,9 @@ def test_warm_start_inside_the_captured_solve(gpu, cupf, syn):
 
 
 @pytest.mark.parametrize("compute", ["Mixed", "FP64"])
-def test_batch_one_graph(gpu, cupf, syn, compute):
-    """Batch 1 runs the single-system kernels inside the captured solve."""
-    g = syn.workload_grid("case118")
+def test_batch_one_graph(gpu, cupf, syn, grid, compute):
+    """Batch 1: the whole loop in one launch, or the level sweeps of one scenario."""
+    g = grid
     eager = _solver(cupf, g, compute, False)
     graph = _solver(cupf, g, compute, True)
     args = (g.indptr, g.indices, g.data, g.n_bus, g.n_bus)

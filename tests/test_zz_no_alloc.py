@@ -49,11 +49,23 @@ def _static(lib, h, torch, vals, rhs, transpose):
     return d_x.cpu().numpy()
 
 
+@pytest.fixture(params=[118, 400])
+def system(request, syn, oracle):
+    """A Jacobian that one workgroup factors, and one that the level sweeps do."""
+    if request.param == 118:
+        return _golden("case118")
+    g = syn.make_grid(400, 620, 60, seed=400, load_scale=0.25)
+    ja = oracle.jacobian_analysis(g.n_bus, g.indptr, g.indices, g.pv, g.pq)
+    vals = oracle.jacobian_values(g.n_bus, g.indptr, g.indices, g.data, g.flat_start(), g.pv, g.pq, ja["nnz"])
+    A = scipy.sparse.csr_matrix((vals, ja["col_idx"], ja["row_ptr"]), shape=(ja["dim"],) * 2)
+    return A, np.random.default_rng(9).standard_normal(ja["dim"])
+
+
 @pytest.mark.parametrize("precision,cap,refine", [(0, 8, 0), (1, 64, 2)])
-def test_static_matches_allocating_entry(gpu, precision, cap, refine):
+def test_static_matches_allocating_entry(gpu, system, precision, cap, refine):
     torch = gpu
     lib = capi.lib()
-    A, b = _golden("case118")
+    A, b = system
     n = A.shape[0]
     cfg = LuConfig()
     lib.cupf_lu_default_config(ctypes.byref(cfg))
@@ -66,9 +78,10 @@ def test_static_matches_allocating_entry(gpu, precision, cap, refine):
         _lu_check(lib.cupf_lu_analyze(h, n, int(A.nnz), rp.ctypes.data_as(ctypes.c_void_p),
                                       ci.ctypes.data_as(ctypes.c_void_p), 0))
         rng = np.random.default_rng(5)
-        # two calls in a row, the second with a smaller batch (128 then 64 lanes)
-        for B, seed, transpose in ((100, 1, False), (7, 2, True)):
-            print(f"[no-alloc] case118 precision={precision} cap={cap} batch={B} "
+        # two calls in a row, the second with a smaller batch (128 then 64 lanes
+        # on 118 buses)
+        for B, seed, transpose in ((100 if n < 400 else 50, 1, False), (7, 2, True)):
+            print(f"[no-alloc] dim={n} precision={precision} cap={cap} batch={B} "
                   f"transpose={transpose}", flush=True)
             vals = _batch_values(A, B, seed)
             rhs = np.vstack([b * rng.uniform(0.5, 1.5, n) for _ in range(B)])
