@@ -260,7 +260,9 @@ void BatchedLU::analyze(int n, const int* rp, const int* ci, const std::vector<i
 // 250 buses mixed (one workgroup per CU): x1,024 2.05 against 3.12 ms, x1,536
 // 3.00 against 3.41, x2,048 4.6 against 3.9; 118 buses mixed (two): x2,048 1.60
 // against 2.38; 30 buses FP64 (seven): x2,048 0.71 against 1.05, x4,096 1.28
-// against 1.16.  The line lies where every measured shape gains.
+// against 1.16.  The line lies where every measured shape gains: also 60 to 450
+// buses with 1.05 to 1.6 branches each, FP64 and mixed, x256 3.6 to 6.1 times as
+// fast as the sweeps, x1,024 1.25 to 3.2 times.
 constexpr int kSysPerCu = 1024, kSysEver = 2048;
 
 void BatchedLU::find_sys(int n_bus, const int* rp, const int* ci, hipStream_t s) {

@@ -1720,21 +1720,26 @@ __global__ __launch_bounds__(kChainThreads, 2) void k_chain_strips(LuDevice d, C
 //     16x16x4, a 16-row strip per wave).
 //   k_schur_tile (one workgroup per (tile, scenario), 256 lanes): one
 //     64 x 64 tile of the contribution block C = A22 - L21 U12.  The tile of
-//     A22 is assembled in LDS (entries, then the tile's chunk map); each wave
-//     then loads its operands (32 rows of L21, 32 columns of U12) and forms
+//     A22 is assembled in LDS (the tile's chunk map; the matrix's entries lie
+//     in pivot rows and columns); each wave then loads its operands (32 rows of
+//     L21, 32 columns of U12) and forms
 //     its 32 x 32 quarter on MFMA (FP32 32x32x2, 3xBF16 32x32x16, or FP64
 //     16x16x4 as 2 x 2 tiles, eight pivots of a lane at a time) starting from
 //     the assembled values, and writes it once.  Loads return in order, so
 //     operands requested before the assembly would delay its loads; without
 //     them FP64 takes 113 VGPRs (four workgroups per CU).
-//     Bound by the assembly's chain of dependent loads (chunk, child element,
-//     LDS) in a workgroup's 20 to 40 us, four to a CU.  2,000 buses x 1,024,
-//     FP64: the levels with at most 32 pivots went from 2.18, 1.05, 0.85 and
-//     0.50 to 1.48, 0.69, 0.54 and 0.28 ms; those with 64 lost a tenth (1.17
-//     to 1.30, 0.81 to 0.92 ms), and the solve went from 97.0 to 84.6 ms with
-//     the other tier-2 kernels.  A form with all 64 pivots' operands in
+//     What bounds it depends on the pivots (FP64 on 2,000 buses x 1,024, copies
+//     without one part or the other): on a level with at most 25 pivots the
+//     assembly's chain of dependent loads is 27-32 % of the launch and the
+//     operands' loads 13-16 %; on a 443-row front with 64 pivots 26 % and 42 %
+//     (1.35 ms; 1.00 without the assembly, 0.78 without the operands, 0.41
+//     without both), on a 187-row one 15 % and 53 %.  So the levels with few
+//     pivots went from 0.50, 2.07 and 2.38 ms to 0.32, 1.33 and 1.67 with the
+//     operands behind the assembly, and those with 64 lost 4 to 20 % (2.10 to
+//     2.18, 1.23 to 1.35, 0.85 to 0.96 ms); the solve went from 97.0 to 84.6 ms
+//     with the other tier-2 kernels.  A form with all 64 pivots' operands in
 //     registers for the groups that need them, at three workgroups per CU,
-//     did not bring the tenth back.
+//     did not bring the loss back.
 //
 // The operands' k index is split by lane group so every lane reads a run of
 // kw contiguous L21 elements, kw being the pivots dealt to a group (K over

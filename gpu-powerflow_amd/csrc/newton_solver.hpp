@@ -105,7 +105,10 @@ public:
     // HIP-event timing of the stages on the stream they run on.
     // Stage order: residual, jacobian, factor, solve (with refinement),
     // voltage update, dense-front factor launches (nested in factor), warm
-    // start.  collect_stage_times() synchronises and resets.
+    // start.  collect_stage_times() synchronises and resets.  While it is on,
+    // small grids run the stages as launches of their own (one workgroup per
+    // scenario factors and solves) instead of whole Newton steps in one launch:
+    // the stage times are of those launches.
     void set_stage_timing(bool on);
     void collect_stage_times(double* total_ms, int64_t* launches);
 

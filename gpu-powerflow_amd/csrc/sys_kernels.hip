@@ -12,11 +12,13 @@
 // whole workgroup, the front's elements in registers and the pivot row and
 // column passed through LDS.
 //
-// What bounds it is the chain of dependent instructions (a wave alone on its
-// SIMD issues one about every 9 cycles): on 118 buses FP64 a Newton step takes
-// 69 us, 45 of them the 43 + 20 pivots of its levels one after another, 16 the
-// solve.  Solves: 118 buses x1 FP64 1.92 -> 0.40 ms (captured mixed 1.67 ->
-// 0.33), x300 mixed 2.73 -> 0.48, x1,024 FP64 3.14 -> 1.41.
+// What bounds it is latency: on 118 buses FP64 a Newton step takes 72 us, 30 of
+// them the 43 pivots of the shared fronts one after another (0.7 us each, with
+// one barrier and, per thread, the update of 8 elements), 13 the levels of quads
+// and wave fronts, 20 the solve, 4.5 the residual and stop test (a wave alone on
+// its SIMD issues an instruction about every 9 cycles).  Solves: 118 buses x1
+// FP64 1.92 -> 0.41 ms (captured mixed 1.67 -> 0.34), x300 mixed 2.73 -> 0.50,
+// x1,024 FP64 3.14 -> 1.46.
 #include "sys_kernels.hpp"
 #include "hip_common.hpp"
 

@@ -217,7 +217,8 @@ int cupf_solver_solve_batch_device_ybus(cupf_solver* solver, const void* sbus,
                                         int32_t* iterations, double* final_mismatch,
                                         uint8_t* converged, void* stream);
 
-/* HIP-event stage timing (no reference counterpart; the reference's
+/* HIP-event stage timing (small grids run their stages as separate launches
+ * while it is on, see set_stage_timing in newton_solver.hpp; no reference counterpart; the reference's
  * ENABLE_TIMING ScopedTimer, utils/timer.hpp:52-283, syncs per stage).
  * Stages: 0 residual, 1 jacobian, 2 factor, 3 solve+refine, 4 voltage update,
  * 5 dense-front (tier-2) factor launches, nested inside 2, 6 warm start.
