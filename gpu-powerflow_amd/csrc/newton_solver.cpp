@@ -359,6 +359,11 @@ struct NewtonSolver::Impl {
     // launch on a stopped control word returns at once (2-3 us), a readback
     // costs 15-20 us.
     static constexpr int kSysAhead = 4;
+    // Most steps of one launch on one scenario (some 2 ms): a scenario that
+    // neither converges nor diverges comes back to the host now and then,
+    // whatever max_iter is.  A solve takes 4 to 10.
+    static constexpr int kSysAlone = 32;
+    int alone_steps(int limit) const { return B == 1 ? std::min(limit - 1, kSysAlone) : 0; }
 
     // Eager loop on the one-workgroup kernel; the order and the outcome of
     // the loop above, with one readback for several steps.
@@ -366,12 +371,12 @@ struct NewtonSolver::Impl {
         if (head) head();
         int c[5] = {0, 0, 0, 0, 0};
         double m = 0.0;
-        sys_launch(cfg, tolerant, limit, true, B == 1 ? limit - 1 : 0);
+        sys_launch(cfg, tolerant, limit, true, alone_steps(limit));
         for (int k = 0; B > 1 && k < std::min(kSysAhead, limit - 1); ++k)
             sys_launch(cfg, tolerant, limit, false, 1);
         read_control(c, m);
         while (!c[0]) {
-            sys_launch(cfg, tolerant, limit, false, 1);
+            sys_launch(cfg, tolerant, limit, false, std::max(1, alone_steps(limit)));
             read_control(c, m);
         }
         st.factorizations += c[2] - 1;
@@ -390,7 +395,7 @@ struct NewtonSolver::Impl {
                    int limit) {
         if (head) head();
         if (sys_loop()) {
-            sys_launch(cfg, tolerant, limit, true, B == 1 ? limit - 1 : 0);
+            sys_launch(cfg, tolerant, limit, true, alone_steps(limit));
             return;
         }
         eval_residual();
@@ -406,7 +411,7 @@ struct NewtonSolver::Impl {
     // stop test from running when the device wants refinement.
     void loop_step(const NRConfig& cfg, bool tolerant, int limit, bool refined) {
         if (sys_loop()) {                 // refined as the control word says
-            sys_launch(cfg, tolerant, limit, false, 1);
+            sys_launch(cfg, tolerant, limit, false, std::max(1, alone_steps(limit)));
             return;
         }
         refined = refined && refine > 0;
@@ -489,7 +494,7 @@ struct NewtonSolver::Impl {
             if (head_id) head_warm = head_id;
         } else {
             // the one-workgroup launches decide on the refinement themselves, and
-            // one scenario's first launch runs the whole loop
+            // one scenario's first launch runs the loop as far as kSysAlone steps
             const bool sys = sys_loop();
             const int steps = sys && B == 1 ? 0 : std::min(pred_steps[ti], limit - 1);
             const unsigned pattern =

@@ -208,3 +208,28 @@ def test_pivots_at_the_ends_of_the_range(gpu, precision, tiny, huge, rows):
     assert not flags.any()
     np.testing.assert_array_equal(x, want)
     np.testing.assert_array_equal(xt, want)
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_one_scenario_that_does_not_converge(gpu, cupf, syn, graph):
+    """A tolerance of zero: the loop ends at the limit, 100 evaluations, with the
+    same state as the level sweeps' (2,049 scenarios) and, captured, after more
+    than one launch, so no launch is as long as the limit."""
+    g = _grid(syn, 30)
+    S = g.sbus_scaled(syn.load_factors(2049, 30, 0.7, 1.3, 6))
+    V0 = g.flat_start(2049)
+    args = (g.indptr, g.indices, g.data, 30, 30)
+    c = cupf.NRConfig()
+    c.tolerance, c.max_iter = 0.0, 100
+    o = cupf.NewtonOptions()
+    o.compute, o.use_cuda_graph = cupf.ComputePolicy.FP64, graph
+    s = cupf.NewtonSolver(o)
+    s.initialize(g.indptr, g.indices, g.data, 30, 30, g.pv, g.pq)
+    many = s.solve_batch(*args, S, V0, g.pv, g.pq, c)
+    for call in range(3):
+        before = s.stats()["graph_launches"]
+        one = s.solve_batch(*args, S[:1], V0[:1], g.pv, g.pq, c)
+        assert one.iterations_numpy[0] == many.iterations_numpy[0] == 100
+        np.testing.assert_allclose(one.V_numpy, many.V_numpy[:1], rtol=0, atol=1e-12)
+        launches = s.stats()["graph_launches"] - before
+        assert launches == (0 if not graph or call == 0 else 4)     # 32 + 32 + 32 + 3 steps
