@@ -18,7 +18,7 @@
 // and wave fronts, 20 the solve, 4.5 the residual and stop test (a wave alone on
 // its SIMD issues an instruction about every 9 cycles).  Solves: 118 buses x1
 // FP64 1.92 -> 0.41 ms (captured mixed 1.67 -> 0.34), x300 mixed 2.73 -> 0.50,
-// x1,024 FP64 3.14 -> 1.46.
+// x1,024 FP64 3.14 -> 1.44.
 #include "sys_kernels.hpp"
 #include "hip_common.hpp"
 
@@ -30,38 +30,21 @@ namespace {
 
 constexpr unsigned long long kNanBits = 0x7FF8000000000000ULL;
 
-// Pivots from least() up to most() have a reciprocal that is a normal number.
-__device__ __forceinline__ double least(double) { return 0x1p-1022; }
-__device__ __forceinline__ double most(double) { return 0x1p1022; }
-__device__ __forceinline__ float least(float) { return 0x1p-126f; }
-__device__ __forceinline__ float most(float) { return 0x1p126f; }
-
 // The pivot rule of the batched kernels without branches: |pivot| <= low
 // becomes +-rep and raises the flag (static pivots: both are eps; else a zero
-// pivot becomes 1).  Plain pivots are not replaced and have a reciprocal.
+// pivot becomes 1).
 template <typename T>
 struct PivotRule {
-    T low, rep, floor;
+    T low, rep;
     bool sign;
     __device__ __forceinline__ PivotRule(double eps, int static_piv)
-        : low(static_piv ? T(eps) : T(0)), rep(static_piv ? T(eps) : T(1)),
-          floor(low > least(T()) ? low : least(T())), sign(static_piv != 0) {}
+        : low(static_piv ? T(eps) : T(0)), rep(static_piv ? T(eps) : T(1)), sign(static_piv != 0) {}
     __device__ __forceinline__ bool small(T piv) const { return (piv < T(0) ? -piv : piv) <= low; }
     __device__ __forceinline__ T replaced(T piv) const { return sign && piv < T(0) ? -rep : rep; }
-    __device__ __forceinline__ bool plain(T piv) const {
-        const T m = piv < T(0) ? -piv : piv;
-        return m > floor && m < most(T());
-    }
-    // piv, or NaN (which the reciprocal hands on to the solves' quotients)
-    // where it has no reciprocal
-    __device__ __forceinline__ T divisor(T piv) const {
-        const T m = piv < T(0) ? -piv : piv;
-        return m >= least(T()) && m < most(T()) ? piv : T(__builtin_nanf(""));
-    }
 };
 
-// 1 / d by Newton's iteration from the hardware estimate, within an ulp; NaN
-// for NaN.
+// 1 / d by Newton's iteration from the hardware estimate, within an ulp where it
+// is a normal number, else something that is not.
 __device__ __forceinline__ double reciprocal(double d) {
     double r = __builtin_amdgcn_rcp(d);
     r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
@@ -74,9 +57,9 @@ __device__ __forceinline__ float reciprocal(float d) {
 
 // a / d from r = 1 / d: the product and one residual correction, which round
 // as the division does (no difference in 10^8 pairs of either type) at a
-// quarter of its latency.  NaN where r is NaN, a is infinite or the quotient
-// overflows: the factorisations look at their pivots, the solves at their
-// results, and divide then.
+// quarter of its latency.  No number where r is none, a is infinite or the
+// quotient overflows: a factorisation looks at its reciprocals, a solve at its
+// results, and both start again by division then (factor_matrix, solve_system).
 __device__ __forceinline__ double quotient(double a, double d, double r) {
     const double q = a * r;
     return __builtin_fma(__builtin_fma(-d, q, a), r, q);
@@ -125,6 +108,7 @@ __device__ __forceinline__ void wave_sync() {
 // Pivot row and column buffers: a share for each of eight waves, or all of
 // them for a shared front.
 constexpr int kWaveBuf = 128, kSysBuf = 8 * kWaveBuf;
+constexpr int kSysMark = 4;           // elements of Sys::mark (16 or 32 bytes)
 
 // The tables and arrays of one system in LDS.  `a` holds the factors at 0 and
 // the scratch region (contribution blocks, then work vectors) at scr.
@@ -134,6 +118,7 @@ struct Sys {
     T* dinv;
     T* y;
     T* buf;                           // the front teams' pivot rows and columns
+    int* mark;                        // see any_thread()
     int scr;
     const SysFront* front;
     const int* level;
@@ -279,31 +264,6 @@ __device__ __forceinline__ int over_groups(int v) {
                max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
 }
 
-// The same by division on the assembled fronts in LDS, for fronts with a pivot
-// that has no reciprocal.
-template <typename T>
-__device__ __forceinline__ void eliminate_dividing(const Sys<T>& S, const Front& f, int r, int fs, int K,
-                                                   int kmax, const PivotRule<T>& rule, int& flag) {
-    for (int k = 0; k < kmax; ++k) {
-        const bool on = k < K, below = on && r > k && r < fs;
-        T piv = on ? S.a[f.at(k, k)] : T(1);
-        const bool low = on && rule.small(piv);
-        flag |= low;
-        piv = low ? rule.replaced(piv) : piv;
-        wave_sync();
-        if (on && r == k) {
-            S.a[f.at(k, k)] = piv;
-            S.dinv[f.first + k] = reciprocal(rule.divisor(piv));
-        }
-        if (below) {
-            const T l = S.a[f.at(r, k)] / piv;
-            S.a[f.at(r, k)] = l;
-            for (int j = k + 1; j < fs; ++j) S.a[f.at(r, j)] = nfma(l, S.a[f.at(k, j)], S.a[f.at(r, j)]);
-        }
-        wave_sync();
-    }
-}
-
 // Four fronts of at most 16 rows, one per 16 lanes: contribution blocks added
 // in LDS, the rows factored in registers.
 template <typename T>
@@ -331,13 +291,7 @@ __device__ __forceinline__ void factor_quad(const Sys<T>& S, const unsigned shor
         x[j] = r < fs && j < fs ? v : T(0);
     }
     T rinv = T(1);
-    int replaced = 0;
-    eliminate16<0>(x, r, K, kmax, rule, replaced, rinv);
-    if (__builtin_expect(__any(!__builtin_isnormal(rinv)), 0)) {
-        eliminate_dividing(S, f, r, fs, K, kmax, rule, flag);
-        return;
-    }
-    flag |= replaced;
+    eliminate16<0>(x, r, K, kmax, rule, flag, rinv);
 #pragma unroll
     for (int j = 0; j < 16; ++j)
         if (r < fs && j < fs) S.a[(j < f.K ? lo : hi) + j] = x[j];
@@ -404,23 +358,18 @@ __device__ __forceinline__ void factor_front(const Sys<T>& S, int p, T* buf, con
 #pragma unroll
                 for (int a = 0; a < RA; ++a) c[a] = cb[ti + TR * a];
                 const T my_c = cb[mine], my_u = rb[mine];
-                T r = reciprocal(piv);
+                if (__builtin_expect(__any(rule.small(piv)), 0)) {      // the same for all
+                    flag = 1;
+                    piv = rule.replaced(piv);
+                }
+                const T r = reciprocal(piv);
                 // column / pivot as the column times the reciprocal and its
                 // error, one rounding: an instruction a quotient less
                 const T rerr = nfma(piv, r, T(1)) * r;
-                T l[RA], my_l = mul_add(r, my_c, my_c * rerr);
+                const T my_l = mul_add(r, my_c, my_c * rerr);
+                T l[RA];
 #pragma unroll
                 for (int a = 0; a < RA; ++a) l[a] = mul_add(r, c[a], c[a] * rerr);
-                if (__builtin_expect(__any(!rule.plain(piv)), 0)) {     // the same for all
-                    if (rule.small(piv)) {
-                        flag = 1;
-                        piv = rule.replaced(piv);
-                    }
-                    r = reciprocal(rule.divisor(piv));
-                    my_l = my_c / piv;
-#pragma unroll
-                    for (int a = 0; a < RA; ++a) l[a] = c[a] / piv;
-                }
 #pragma unroll
                 for (int a = 0; a < RA; ++a)
 #pragma unroll
@@ -465,6 +414,100 @@ __device__ __forceinline__ void factor_system(const Sys<T>& S, double eps, int s
             else factor_front<T, kSysMaxRows / 16, (kSysMaxRows * 16 + NT - 1) / NT, 16, NT / 16, true>(S, p, S.buf, rule, flag);
         }
     }
+}
+
+// One front by one wave, in LDS and by division.
+template <typename T>
+__device__ __forceinline__ void factor_dividing(const Sys<T>& S, int p, const PivotRule<T>& rule, int& flag) {
+    const int lane = int(threadIdx.x) & 63;
+    const Front f = load_front(S, p);
+    for (int e = lane; e < f.uc * f.uc; e += 64) S.a[f.co + e] = T(0);
+    wave_sync();
+    add_children(S, f, lane >> 4, 4);
+    wave_sync();
+    for (int k = 0; k < f.K; ++k) {
+        T piv = S.a[f.at(k, k)];
+        if (rule.small(piv)) {
+            flag = 1;
+            piv = rule.replaced(piv);
+        }
+        wave_sync();
+        if (lane == 0) {
+            const T r = reciprocal(piv);
+            S.a[f.at(k, k)] = piv;
+            S.dinv[f.first + k] = __builtin_isnormal(r) ? r : T(__builtin_nanf(""));    // the solves divide
+        }
+        for (int i = k + 1 + lane; i < f.fs; i += 64) {
+            const T l = S.a[f.at(i, k)] / piv;
+            S.a[f.at(i, k)] = l;
+            for (int j = k + 1; j < f.fs; ++j) S.a[f.at(i, j)] = nfma(l, S.a[f.at(k, j)], S.a[f.at(i, j)]);
+        }
+        wave_sync();
+    }
+}
+
+// All fronts so.  A function of its own, as divide_solve(): inlined, their
+// registers and code slow the plain path by 1-4%.
+template <typename T>
+__device__ __attribute__((noinline)) int divide_factors(T* a, T* dinv, int scr, const SysFront* front, const int* level,
+                                                        const int* slice, const unsigned short* list,
+                                                        const unsigned short* adds, int o_task, int num_levels,
+                                                        double eps, int static_piv) {
+    Sys<T> S{};
+    S.a = a;
+    S.dinv = dinv;
+    S.scr = scr;
+    S.front = front;
+    S.level = level;
+    S.slice = slice;
+    S.list = list;
+    S.adds = adds;
+    const PivotRule<T> rule(eps, static_piv);
+    int flag = 0;
+    for (int L = 0; L < num_levels; ++L) {
+        const int* lv = level + L * kSysLevelInts;
+        const unsigned short* task = list + o_task + lv[0];
+        for (int t = int(threadIdx.x) >> 6; t < lv[2] + 4 * lv[1] + lv[3]; t += int(blockDim.x) >> 6)
+            if (task[t] != 0xffff) factor_dividing(S, task[t], rule, flag);
+        __syncthreads();
+    }
+    return flag;
+}
+
+// Back to 0 once every thread has read it.
+template <typename T>
+__device__ __forceinline__ void clear_mark(const Sys<T>& S) {
+    __syncthreads();
+    if (threadIdx.x == 0) *S.mark = 0;
+    __syncthreads();
+}
+
+// Whether `yes` holds on any thread of the workgroup (one barrier).  S.mark is 0
+// before and after; two calls have a barrier between them.
+template <typename T>
+__device__ __forceinline__ bool any_thread(const Sys<T>& S, bool yes) {
+    if (yes) *S.mark = 1;
+    __syncthreads();
+    if (__builtin_expect(*S.mark == 0, 1)) return false;
+    clear_mark(S);
+    return true;
+}
+
+// The factors of the matrix that load() puts into the factors' place (it ends
+// with a barrier).  A pivot whose reciprocal is no normal number has it all done
+// again by division, unless hopeless() finds a NaN among this thread's inputs.
+template <typename T, int NT, class F, class G>
+__device__ __forceinline__ void factor_matrix(const Sys<T>& S, int n, double eps, int static_piv, int& flag,
+                                              F load, G hopeless) {
+    load();
+    factor_system<T, NT>(S, eps, static_piv, flag);
+    bool normal = true;
+    for (int k = int(threadIdx.x); k < n; k += NT) normal = normal && __builtin_isnormal(S.dinv[k]);
+    if (!any_thread(S, !normal) || any_thread(S, hopeless())) return;
+    flag = 0;
+    load();
+    flag = divide_factors(S.a, S.dinv, S.scr, S.front, S.level, S.slice, S.list, S.adds, S.o_task, S.num_levels,
+                          eps, static_piv);
 }
 
 // Solve sweeps on y (permuted order).  Fronts of at most 16 rows four to a
@@ -626,8 +669,36 @@ __device__ __forceinline__ void sweep_system(const Sys<T>& S) {
     }
 }
 
-// y = A^-1 y (or A^-T y).  A result that is not finite is computed again by
-// division: load() puts the right-hand side into y.
+template <bool TRANS, typename T>
+__device__ __attribute__((noinline)) void divide_solve(T* a, T* dinv, T* y, int scr, const SysFront* front,
+                                                       const int* level, const unsigned short* list, int o_task,
+                                                       int o_rows, int o_gptr, int o_gsrc, int num_levels) {
+    Sys<T> S{};
+    S.a = a;
+    S.dinv = dinv;
+    S.y = y;
+    S.scr = scr;
+    S.front = front;
+    S.level = level;
+    S.list = list;
+    S.o_task = o_task;
+    S.o_rows = o_rows;
+    S.o_gptr = o_gptr;
+    S.o_gsrc = o_gsrc;
+    S.num_levels = num_levels;
+    sweep_system<TRANS, true>(S);
+}
+
+// On this thread's elements.
+template <typename T>
+__device__ __forceinline__ bool factors_hold_nan(const Sys<T>& S) {
+    bool nan = false;
+    for (int e = int(threadIdx.x); e < S.scr; e += int(blockDim.x)) nan = nan || S.a[e] != S.a[e];
+    return nan;
+}
+
+// y = A^-1 y (or A^-T y); load() puts the right-hand side into y.  A result that
+// is not finite is computed again by division, unless the factors hold a NaN.
 template <bool TRANS, typename T, class F>
 __device__ __forceinline__ void solve_system(const Sys<T>& S, int n, F load) {
     load();
@@ -635,10 +706,12 @@ __device__ __forceinline__ void solve_system(const Sys<T>& S, int n, F load) {
     sweep_system<TRANS, false>(S);
     bool finite = true;
     for (int k = int(threadIdx.x); k < n; k += int(blockDim.x)) finite = finite && __builtin_isfinite(S.y[k]);
-    if (__builtin_expect(__syncthreads_or(!finite), 0)) {
+    if (any_thread(S, !finite)) {
+        if (any_thread(S, factors_hold_nan(S))) return;
         load();
         __syncthreads();
-        sweep_system<TRANS, true>(S);
+        divide_solve<TRANS>(S.a, S.dinv, S.y, S.scr, S.front, S.level, S.list, S.o_task, S.o_rows, S.o_gptr, S.o_gsrc,
+                            S.num_levels);
     }
 }
 
@@ -657,14 +730,18 @@ __device__ __forceinline__ unsigned char* carve(const SysDevice& d, unsigned cha
     S.scr = d.fac;
     S.dinv = take(d.n);
     S.y = take(d.n);
-    S.buf = take(kSysBuf);
+    S.buf = take(kSysBuf + kSysMark);
+    S.mark = reinterpret_cast<int*>(S.buf + kSysBuf);
     int4* blob = reinterpret_cast<int4*>(at);
     for (int e = int(threadIdx.x); e < d.blob_quads; e += int(blockDim.x)) blob[e] = d.blob[e];
     const int* ints = reinterpret_cast<const int*>(at);
     S.front = reinterpret_cast<const SysFront*>(ints);
     S.level = ints + d.o_level;
     S.list = reinterpret_cast<const unsigned short*>(ints);
-    if (threadIdx.x == 0) S.a[d.fac + d.scratch - 1] = T(0);   // the zero element
+    if (threadIdx.x == 0) {
+        S.a[d.fac + d.scratch - 1] = T(0);                      // the zero element
+        *S.mark = 0;
+    }
     S.slice = ints + d.o_slice;
     S.adds = d.adds;
     S.o_task = d.o_task;
@@ -684,25 +761,29 @@ __global__ __launch_bounds__(NT, 2) void k_sys_factor(SysDevice d, const double*
     Sys<T> S;
     carve(d, smem, S);
     const int b = blockIdx.x, tid = threadIdx.x;
-    for (int e = tid; e < d.fac; e += NT) S.a[e] = T(0);
-    __syncthreads();
-    for (int k0 = tid; k0 < d.nnz; k0 += 4 * NT) {
-        int at[4];
-        double v[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int k = min(k0 + u * NT, d.nnz - 1);
-            at[u] = d.slot_pos[k];
-            v[u] = A[(long long)k * Bp + b];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (k0 + u * NT < d.nnz) S.a[at[u]] = T(v[u]);
-    }
-    __syncthreads();
     int flag = 0;
-    factor_system<T, NT>(S, eps, static_piv, flag);
-    __syncthreads();
+    factor_matrix<T, NT>(S, d.n, eps, static_piv, flag, [&] {
+        for (int e = tid; e < d.fac; e += NT) S.a[e] = T(0);
+        __syncthreads();
+        for (int k0 = tid; k0 < d.nnz; k0 += 4 * NT) {
+            int at[4];
+            double v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int k = min(k0 + u * NT, d.nnz - 1);
+                at[u] = d.slot_pos[k];
+                v[u] = A[(long long)k * Bp + b];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (k0 + u * NT < d.nnz) S.a[at[u]] = T(v[u]);
+        }
+        __syncthreads();
+    }, [&] {
+        bool nan = false;
+        for (int k = tid; k < d.nnz; k += NT) nan = nan || __builtin_isnan(A[(long long)k * Bp + b]);
+        return nan;
+    });
     T* out = store + (long long)b * (d.fac + d.n);
     for (int e = tid; e < d.fac; e += NT) out[e] = S.a[e];
     for (int e = tid; e < d.n; e += NT) out[d.fac + e] = S.dinv[e];
@@ -923,30 +1004,38 @@ __global__ __launch_bounds__(NT, 2) void k_sys_newton(SysDevice d, NrDevice nr, 
         else __syncthreads();
         if (pass == o.steps || word[0]) break;
         const int solves = word[1] ? 1 : 1 + o.refine;
-        for (int e = tid; e < d.fac; e += NT) S.a[e] = T(0);
-        __syncthreads();
-        for (int k = tid; k < nr.nnzY; k += NT) {
-            const int4 at4 = net.ydst[k];
-            double2 dva, dvm;
-            entry_jacobian(n, y_value(nr, k, Bp, b), net.yrow[k], nr.yi[k], dva, dvm);
-            if (at4.x >= 0) S.a[at4.x] = T(dva.x);
-            if (at4.y >= 0) S.a[at4.y] = T(dva.y);
-            if (at4.z >= 0) S.a[at4.z] = T(dvm.x);
-            if (at4.w >= 0) S.a[at4.w] = T(dvm.y);
-        }
-        __syncthreads();
+        auto load_jacobian = [&] {
+            for (int e = tid; e < d.fac; e += NT) S.a[e] = T(0);
+            __syncthreads();
+            for (int k = tid; k < nr.nnzY; k += NT) {
+                const int4 at4 = net.ydst[k];
+                double2 dva, dvm;
+                entry_jacobian(n, y_value(nr, k, Bp, b), net.yrow[k], nr.yi[k], dva, dvm);
+                if (at4.x >= 0) S.a[at4.x] = T(dva.x);
+                if (at4.y >= 0) S.a[at4.y] = T(dva.y);
+                if (at4.z >= 0) S.a[at4.z] = T(dvm.x);
+                if (at4.w >= 0) S.a[at4.w] = T(dvm.y);
+            }
+            __syncthreads();
+        };
+        const unsigned short* perm = S.list + S.o_perm;
+        load_jacobian();
         int flag = 0;
         factor_system<T, NT>(S, eps, static_piv, flag);
-        if (flag) atomicOr(sing + b, 1);
+        // As factor_matrix() and solve_system(), with the reciprocals and results
+        // looked at on the way and told over the barriers that are there anyway:
+        // kLook until one asks for divisions, then kDivide, or kLeave where there
+        // is a NaN
+        enum { kLook, kLeave, kDivide } mode = kLook;
         for (int it = 0; it < solves; ++it) {
             // refinement: F - J dx, a bus's two rows per thread; the mismatch
             // itself is formed again from the row currents (F then holds the
-            // residual)
-            for (int i = tid; it > 0 && i < nr.n_bus; i += NT) {
+            // residual), as it is to start the solves again
+            for (int i = tid; (it > 0 || mode == kDivide) && i < nr.n_bus; i += NT) {
                 const int r1 = nr.row_pvpq[i], r2 = nr.row_pq[i];
                 if (r1 < 0) continue;
                 double ap = 0.0, aq = 0.0;
-                for (int k = nr.yp[i]; k < nr.yp[i + 1]; ++k) {
+                for (int k = nr.yp[i]; it > 0 && k < nr.yp[i + 1]; ++k) {
                     const int j = nr.yi[k];
                     double2 dva, dvm;
                     entry_jacobian(n, y_value(nr, k, Bp, b), i, j, dva, dvm);
@@ -960,14 +1049,44 @@ __global__ __launch_bounds__(NT, 2) void k_sys_newton(SysDevice d, NrDevice nr, 
                 if (r2 >= 0) n.F[r2] = fi.y - aq;
             }
             __syncthreads();
-            const unsigned short* perm = S.list + S.o_perm;
-            solve_system<false>(S, d.n, [&] {
-                for (int k = tid; k < d.n; k += NT) S.y[k] = T(n.F[perm[k]]);
-            });
-            for (int k = tid; k < d.n; k += NT)
-                n.dx[perm[k]] = it > 0 ? n.dx[perm[k]] + double(S.y[k]) : double(S.y[k]);
+            bool ask = false;
+            for (int k = tid; k < d.n; k += NT) {
+                S.y[k] = T(n.F[perm[k]]);
+                ask = ask || !__builtin_isnormal(S.dinv[k]);
+            }
+            if (ask && mode == kLook) *S.mark = 1;
             __syncthreads();
+            if (__builtin_expect(*S.mark, 0)) {                 // before the first solve, or never
+                clear_mark(S);
+                bool nan = false;
+                for (int i = tid; i < nr.n_bus; i += NT) nan = nan || n.V[i].x != n.V[i].x || n.V[i].y != n.V[i].y;
+                mode = any_thread(S, nan) ? kLeave : kDivide;
+                if (mode == kDivide) {
+                    load_jacobian();
+                    flag = divide_factors(S.a, S.dinv, S.scr, S.front, S.level, S.slice, S.list, S.adds, S.o_task,
+                                          S.num_levels, eps, static_piv);
+                }
+            }
+            if (__builtin_expect(mode == kDivide, 0))
+                divide_solve<false>(S.a, S.dinv, S.y, S.scr, S.front, S.level, S.list, S.o_task, S.o_rows, S.o_gptr,
+                                    S.o_gsrc, S.num_levels);
+            else
+                sweep_system<false, false>(S);
+            ask = false;
+            for (int k = tid; k < d.n; k += NT) {
+                const T y = S.y[k];
+                ask = ask || !__builtin_isfinite(y);
+                n.dx[perm[k]] = it > 0 ? n.dx[perm[k]] + double(y) : double(y);
+            }
+            if (ask && mode == kLook) *S.mark = 1;
+            __syncthreads();
+            if (__builtin_expect(*S.mark, 0)) {
+                clear_mark(S);
+                mode = any_thread(S, factors_hold_nan(S)) ? kLeave : kDivide;
+                if (mode == kDivide) it = -1;                   // the solves again
+            }
         }
+        if (flag) atomicOr(sing + b, 1);
         for (int i = tid; i < nr.n_bus; i += NT) {
             const long long g = (long long)i * Bp + b;
             const int r1 = nr.row_pvpq[i], r2 = nr.row_pq[i];
@@ -996,7 +1115,7 @@ constexpr int kSysCus = 256;
 
 size_t sys_lds_bytes(const SysPlan& p, int elem, int n_bus) {
     auto up = [](size_t v) { return (v + 15) / 16 * 16; };
-    size_t t = up(size_t(p.fac + p.scratch) * elem) + 2 * up(size_t(p.n) * elem) + kSysBuf * size_t(elem) +
+    size_t t = up(size_t(p.fac + p.scratch) * elem) + 2 * up(size_t(p.n) * elem) + (kSysBuf + kSysMark) * size_t(elem) +
                p.blob.size() * sizeof(int);
     if (n_bus > 0) t += size_t(n_bus) * 3 * sizeof(double2) + size_t(p.n) * 2 * sizeof(double);
     return t;

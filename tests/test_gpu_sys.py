@@ -233,3 +233,32 @@ def test_one_scenario_that_does_not_converge(gpu, cupf, syn, graph):
         np.testing.assert_allclose(one.V_numpy, many.V_numpy[:1], rtol=0, atol=1e-12)
         launches = s.stats()["graph_launches"] - before
         assert launches == (0 if not graph or call == 0 else 4)     # 32 + 32 + 32 + 3 steps
+
+
+@pytest.mark.parametrize("compute", ["Mixed", "FP64"])
+@pytest.mark.parametrize("graph", [False, True])
+def test_a_step_whose_pivots_have_no_reciprocal(gpu, cupf, syn, compute, graph):
+    """Two buses, S and Y scaled by a power of two that takes the Jacobian's
+    pivots out of the range of reciprocals (2^1023 in FP64, 2^127 in FP32), so
+    that every step divides: the voltages equal the unscaled grid's, whose steps
+    differ by that power throughout (1e-9: the quotients' rounding near the
+    range's end, over a Jacobian of condition about one)."""
+    g = syn.make_grid(2, 1, 0, seed=2, load_scale=0.25)
+    y = float(np.abs(g.data).max())
+    scale = 2.0 ** ((1023 if compute == "FP64" else 127) - np.floor(np.log2(y)) - 1)
+    V = {}
+    for k in (1.0, scale):
+        o = cupf.NewtonOptions()
+        o.compute = getattr(cupf.ComputePolicy, compute)
+        o.custom.precision = cupf.CustomPrecision.FP64 if compute == "FP64" else cupf.CustomPrecision.FP32
+        o.use_cuda_graph = graph
+        s = cupf.NewtonSolver(o)
+        s.initialize(g.indptr, g.indices, k * g.data, 2, 2, g.pv, g.pq)
+        c = cupf.NRConfig()
+        c.tolerance, c.max_iter = 1e-12 * k, 12
+        S = k * g.sbus_scaled(syn.load_factors(3, 2, 0.7, 1.3, 1))
+        for call in range(2):
+            r = s.solve_batch(g.indptr, g.indices, k * g.data, 2, 2, S, g.flat_start(3), g.pv, g.pq, c)
+            assert r.converged_numpy.all()
+        V[k] = r.V_numpy
+    np.testing.assert_allclose(V[scale], V[1.0], rtol=0, atol=1e-9)
