@@ -446,32 +446,47 @@ __device__ __forceinline__ void factor_dividing(const Sys<T>& S, int p, const Pi
     }
 }
 
+// A pointer into LDS, as the functions below take them: behind a call the
+// compiler could not tell the address space otherwise.
+template <typename X>
+using Lds = __attribute__((address_space(3))) X*;
+template <typename X>
+__device__ __forceinline__ Lds<X> lds(X* p) {
+    return (Lds<X>)p;
+}
+
 // All fronts so.  A function of its own, as divide_solve(): inlined, their
 // registers and code slow the plain path by 1-4%.
 template <typename T>
-__device__ __attribute__((noinline)) int divide_factors(T* a, T* dinv, int scr, const SysFront* front, const int* level,
-                                                        const int* slice, const unsigned short* list,
-                                                        const unsigned short* adds, int o_task, int num_levels,
-                                                        double eps, int static_piv) {
+__device__ __attribute__((noinline)) int divide_factors(Lds<T> a, Lds<T> dinv, int scr, Lds<const int> ints, int o_level,
+                                                        int o_slice, const unsigned short* adds, int o_task,
+                                                        int num_levels, double eps, int static_piv) {
     Sys<T> S{};
-    S.a = a;
-    S.dinv = dinv;
+    S.a = (T*)a;
+    S.dinv = (T*)dinv;
     S.scr = scr;
-    S.front = front;
-    S.level = level;
-    S.slice = slice;
-    S.list = list;
+    S.front = (const SysFront*)(const int*)ints;
+    S.level = (const int*)ints + o_level;
+    S.slice = (const int*)ints + o_slice;
+    S.list = (const unsigned short*)(const int*)ints;
     S.adds = adds;
     const PivotRule<T> rule(eps, static_piv);
     int flag = 0;
     for (int L = 0; L < num_levels; ++L) {
-        const int* lv = level + L * kSysLevelInts;
-        const unsigned short* task = list + o_task + lv[0];
+        const int* lv = S.level + L * kSysLevelInts;
+        const unsigned short* task = S.list + o_task + lv[0];
         for (int t = int(threadIdx.x) >> 6; t < lv[2] + 4 * lv[1] + lv[3]; t += int(blockDim.x) >> 6)
             if (task[t] != 0xffff) factor_dividing(S, task[t], rule, flag);
         __syncthreads();
     }
     return flag;
+}
+
+template <typename T>
+__device__ __forceinline__ int divide_factors(const Sys<T>& S, double eps, int static_piv) {
+    const int* ints = reinterpret_cast<const int*>(S.front);
+    return divide_factors<T>(lds(S.a), lds(S.dinv), S.scr, lds(ints), int(S.level - ints), int(S.slice - ints), S.adds,
+                             S.o_task, S.num_levels, eps, static_piv);
 }
 
 // Back to 0 once every thread has read it.
@@ -506,8 +521,7 @@ __device__ __forceinline__ void factor_matrix(const Sys<T>& S, int n, double eps
     if (!any_thread(S, !normal) || any_thread(S, hopeless())) return;
     flag = 0;
     load();
-    flag = divide_factors(S.a, S.dinv, S.scr, S.front, S.level, S.slice, S.list, S.adds, S.o_task, S.num_levels,
-                          eps, static_piv);
+    flag = divide_factors(S, eps, static_piv);
 }
 
 // Solve sweeps on y (permuted order).  Fronts of at most 16 rows four to a
@@ -670,23 +684,30 @@ __device__ __forceinline__ void sweep_system(const Sys<T>& S) {
 }
 
 template <bool TRANS, typename T>
-__device__ __attribute__((noinline)) void divide_solve(T* a, T* dinv, T* y, int scr, const SysFront* front,
-                                                       const int* level, const unsigned short* list, int o_task,
-                                                       int o_rows, int o_gptr, int o_gsrc, int num_levels) {
+__device__ __attribute__((noinline)) void divide_solve(Lds<T> a, Lds<T> dinv, Lds<T> y, int scr, Lds<const int> ints,
+                                                       int o_level, int o_task, int o_rows, int o_gptr, int o_gsrc,
+                                                       int num_levels) {
     Sys<T> S{};
-    S.a = a;
-    S.dinv = dinv;
-    S.y = y;
+    S.a = (T*)a;
+    S.dinv = (T*)dinv;
+    S.y = (T*)y;
     S.scr = scr;
-    S.front = front;
-    S.level = level;
-    S.list = list;
+    S.front = (const SysFront*)(const int*)ints;
+    S.level = (const int*)ints + o_level;
+    S.list = (const unsigned short*)(const int*)ints;
     S.o_task = o_task;
     S.o_rows = o_rows;
     S.o_gptr = o_gptr;
     S.o_gsrc = o_gsrc;
     S.num_levels = num_levels;
     sweep_system<TRANS, true>(S);
+}
+
+template <bool TRANS, typename T>
+__device__ __forceinline__ void divide_solve(const Sys<T>& S) {
+    const int* ints = reinterpret_cast<const int*>(S.front);
+    divide_solve<TRANS, T>(lds(S.a), lds(S.dinv), lds(S.y), S.scr, lds(ints), int(S.level - ints), S.o_task, S.o_rows,
+                           S.o_gptr, S.o_gsrc, S.num_levels);
 }
 
 // On this thread's elements.
@@ -710,8 +731,7 @@ __device__ __forceinline__ void solve_system(const Sys<T>& S, int n, F load) {
         if (any_thread(S, factors_hold_nan(S))) return;
         load();
         __syncthreads();
-        divide_solve<TRANS>(S.a, S.dinv, S.y, S.scr, S.front, S.level, S.list, S.o_task, S.o_rows, S.o_gptr, S.o_gsrc,
-                            S.num_levels);
+        divide_solve<TRANS>(S);
     }
 }
 
@@ -1063,13 +1083,11 @@ __global__ __launch_bounds__(NT, 2) void k_sys_newton(SysDevice d, NrDevice nr, 
                 mode = any_thread(S, nan) ? kLeave : kDivide;
                 if (mode == kDivide) {
                     load_jacobian();
-                    flag = divide_factors(S.a, S.dinv, S.scr, S.front, S.level, S.slice, S.list, S.adds, S.o_task,
-                                          S.num_levels, eps, static_piv);
+                    flag = divide_factors(S, eps, static_piv);
                 }
             }
             if (__builtin_expect(mode == kDivide, 0))
-                divide_solve<false>(S.a, S.dinv, S.y, S.scr, S.front, S.level, S.list, S.o_task, S.o_rows, S.o_gptr,
-                                    S.o_gsrc, S.num_levels);
+                divide_solve<false>(S);
             else
                 sweep_system<false, false>(S);
             ask = false;
